@@ -20,7 +20,7 @@ Each is checked against the CPU FP64 oracle's columns for this image
 (tests/golden/config_headline.json, matched by the image's SHA-256) and
 against C_ref, FP64 PCG at tolerance 1e-9 on the same image (untimed); a
 result over the metric's 1e-4 is marked invalid and exits non-zero.  The
-cold end-to-end time (hmgInit to C, autotuner included) is reported beside
+cold end-to-end time (hmgInit to C) is reported beside
 the resident-model step time.  The operator kernel of the timed method is timed with HIP
 events on the solver's stream (roofline); the CPU FP64 oracle is timed on a
 bounded sample of the same workload (cpu_baseline).
@@ -299,7 +299,7 @@ def main():
         L.hmgSetHomogenizationFlag(6)
 
     # cold end to end: hmgInit (maps, local matrices) -> upload and solver
-    # allocation -> first homogenization (tile autotuner included) -> C,
+    # allocation -> first homogenization -> C,
     # with the network already trained
     cold = {}
     for label, prec, nt in (("learned_mixed", 1, net), ("plain_fp64", 0, None)):

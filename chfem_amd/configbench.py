@@ -9,8 +9,8 @@ model resident in HBM, one JSON line:
   porosity 0.35 (seed 4), 3 load cases, Jacobi-MINRES to tol 1e-6, FP64 and
   mixed precision.
 
-Each run prepares the model, solves load case 0 once untimed (the autotuner
-and the solver's buffers), then times every load case in turn
+Each run prepares the model, solves load case 0 once untimed (the solver's
+buffers), then times every load case in turn
 (hmgSolveLoadCase) and reports the iterations, refinement sweeps and the
 effective-tensor columns.
 
@@ -44,7 +44,7 @@ def run(L, nf, flat, loads, solver, strategy, precision, tol):
         assert L.hmgPrepare() == 1
         ncol = 6 if loads == 6 else 3
         col = np.zeros(ncol)
-        L.hmgSolveLoadCase(0, None, None, col.ctypes.data_as(C.c_void_p))  # untimed: autotuner, buffers
+        L.hmgSolveLoadCase(0, None, None, col.ctypes.data_as(C.c_void_p))  # untimed: buffers
         cols, its, sweeps, secs, ok = [], [], [], [], []
         st = SolveStats()
         for d in range(loads):

@@ -72,8 +72,8 @@ struct Solver {
     // operator tiles chosen by the autotuner (rows, columns, layers per block)
     bool autotune = false, tuned = false;
     int tile64[3] = {32, 8, 16}, tile32[3] = {32, 8, 16};
-    // CG loop form per precision (see fuse_mode_env), set by the autotuner
-    int mode64 = 1, mode32 = 1;
+    // CG loop form per precision (see fuse_mode_env)
+    int mode64 = 2, mode32 = 2;
     // isotropic elastic materials for the Walsh-basis operator
     double *lamu64 = nullptr;
     float *lamu32 = nullptr;
@@ -212,9 +212,8 @@ static void timed_apply(const OpDesc &op, const T *v, T *q, const Reduce *red)
 // form of the CG loops on the Walsh-basis operators (CHFEM_FUSE_DIR): 0
 // separate operator, direction and update kernels; 1 direction and iterate
 // updates inside the operator, z update kernel; 2 single-kernel iteration,
-// the z update inside the operator too.  Unset or "auto": the autotuner
-// times forms 1 and 2 with every tile and keeps the faster per precision
-// (form 1 when the tiles are fixed).
+// the z update inside the operator too.  Unset or "auto": 2, or what the
+// autotuner measured faster where it runs.
 static int fuse_mode_env()
 {
     const char *e = getenv("CHFEM_FUSE_DIR");
@@ -335,6 +334,7 @@ static cudapcgFlag_t alloc_solver_arrays()
 }
 
 // Build the operator descriptors from the model and the local matrices.
+static bool is_lean();
 static int make_ops()
 {
     cudapcgModel_t *m = g->model;
@@ -359,7 +359,7 @@ static int make_ops()
     o.tile_tc = 8;
     o.tile_lz = 16;
     const char *tile_env = getenv("CHFEM_WALSH_TILE");
-    const bool fixed_tile = tile_env && strcmp(tile_env, "auto") != 0;
+    const bool sweep = tile_env && !strcmp(tile_env, "auto"), fixed_tile = tile_env && !sweep;
     if (fixed_tile) sscanf(tile_env, "%dx%dx%d", &o.tile_tr, &o.tile_tc, &o.tile_lz);
     const char *opsel = getenv("CHFEM_OPERATOR");
     bool use_walsh = g->walsh_ok && !(opsel && !strcmp(opsel, "generic"));
@@ -412,20 +412,26 @@ static int make_ops()
     g->dm.op32.K = g->dm.K32;
     g->dm.op32.lamu = use_walsh ? g->lamu32 : nullptr;
     g->dm.op32.kinv = kj ? g->kinv32 : nullptr;
-    if (!fixed_tile && g->tuned) {
+    if (!fixed_tile && !g->tuned && use_walsh) {
+        const WalshTiles t64 = walsh_tile_rule<double>(o, is_lean()), t32 = walsh_tile_rule<float>(o, is_lean());
+        g->dm.op64.tile_tr = t64.TR; g->dm.op64.tile_tc = t64.TC; g->dm.op64.tile_lz = t64.LZ;
+        g->dm.op32.tile_tr = t32.TR; g->dm.op32.tile_tc = t32.TC; g->dm.op32.tile_lz = t32.LZ;
+    }
+    if (sweep && g->tuned) {
         // tiles picked by the autotuner for this model
         g->dm.op64.tile_tr = g->tile64[0]; g->dm.op64.tile_tc = g->tile64[1]; g->dm.op64.tile_lz = g->tile64[2];
         g->dm.op32.tile_tr = g->tile32[0]; g->dm.op32.tile_tc = g->tile32[1]; g->dm.op32.tile_lz = g->tile32[2];
     }
-    g->autotune = !fixed_tile && use_walsh && !o.ebe;
+    g->autotune = sweep && use_walsh && !o.ebe;
     g->ops_ready = true;
     return 1;
 }
 
-// Operator tile autotuner: times every Walsh tile shape (rows x columns per
-// block, node layers per block) on the model's own grid in each precision the
-// solve uses and keeps the fastest.  Runs once per model, before its first
-// solve; CHFEM_WALSH_TILE=TRxTCxLZ fixes the tile instead.
+// Operator tile autotuner (CHFEM_WALSH_TILE=auto): times Walsh tile shapes
+// (rows x columns per block, node layers per block) and loop forms on the
+// model's own grid in each precision the solve uses and keeps the fastest.
+// Runs once per model, before its first solve.  By default the tile comes
+// from walsh_tile_rule and CHFEM_WALSH_TILE=TRxTCxLZ fixes it.
 static bool is_minres();
 template <typename T> static Ring<T> dir_ring(T *d, T *s, unsigned cap = RING_MAX);
 static void autotune_tiles()
@@ -2018,7 +2024,7 @@ cudapcgFlag_t cudapcgSetLclMtxs(cudapcgVar_t *L)
     // Walsh-basis kernel (per material {lambda, mu} or {k, 0})
     g->walsh_ok = false;
     g->tuned = false;
-    g->mode64 = g->mode32 = 1;
+    g->mode64 = g->mode32 = 2;
     if ((ph == PHY_ELASTIC || ph == PHY_THERMAL) && nk <= 4) {
         double lm[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         float lmf[8];

@@ -271,6 +271,9 @@ namespace chfem {
 // for the unit-voxel trilinear element) and for conduction (lamu: {k, 0} per
 // material, when every local matrix is k times the unit conduction matrix).
 struct WalshTiles { int TR, TC, LZ; };
+// tile and layers per block for the model's grid, from a fitted cost (lean:
+// the memory-lean forms, which run the 32 x 8 tile)
+template <typename T> WalshTiles walsh_tile_rule(const OpDesc &op, int lean);
 template <typename T> struct DirFuse;
 // fz non-null: v is d_old and the launch forms d = z + beta d_old
 // (walsh.h DirFuse), writes it to fz->dnew and reduces d.q (red required).

@@ -2,6 +2,10 @@
 // (device code in walsh.h).
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
+#include <math.h>
+
+#include <algorithm>
+
 #include "walsh.h"
 
 namespace chfem {
@@ -146,6 +150,70 @@ template void launch_walsh_lean<float>(const OpDesc &, int, const float *, float
                                        hipStream_t);
 template void launch_walsh_lean<double>(const OpDesc &, int, const double *, double *, const void *,
                                         const Reduce *, hipStream_t);
+
+// Tile and layers per block of a grid.  What bounds a launch changes with the
+// grid: a block walks its layers one after the other, with two barriers and a
+// load latency per layer, so a grid of few blocks is bound by that chain (a
+// 32^3 FP64 conduction iteration took 24.5 us with 16 layers per block, 12
+// blocks on 256 CUs, and takes 13.9 us with 1 or 2), and a grid of many
+// rounds of blocks by what they load, halos included (256^3 FP32 elastic:
+// 332 us with 65x7x32, 382 us with 32x8x16, 369 us with 65x7x8).  The cost of
+// a candidate in us is
+//   rounds of blocks x (LZ + 2) steps x (d + max(L, work-items on a CU x c))
+//   + h x the values its planes load, every column run rounded up by one
+//     128-byte line,
+// with the CU's resident blocks from the kernels' registers and LDS, and d, L,
+// c, h fitted to timed solves (ring, finishing block and launch gaps
+// included) of cubes of 24 to 256 nodes, a 37x41x56 and a 190x251x233 grid,
+// every tile and LZ 1 to 32.  Over those grids the pick is within 3 % of the
+// fastest candidate, 10 % at the worst, where timing every candidate before
+// the first solve cost as much as 30 (256^3) to 150 (32^3) iterations.
+template <typename T>
+static double tile_cost(const OpDesc &op, int tr, int tc, int lz)
+{
+    const bool dbl = sizeof(T) == 8, el = op.physics == PHY_ELASTIC;
+    static const double fit[2][2][4] = {  // [precision][physics] L, c, d, h
+        {{0.400, 0.00059, 0.337, 1.345}, {0.380, 0.00091, 0.699, 4.266}},
+        {{0.839, 0.00134, 0.000, 1.692}, {0.482, 0.00268, 0.920, 4.836}}};
+    // blocks of 256 and of 512 work-items resident on a CU
+    static const int resident[2][2][2] = {{{8, 4}, {5, 2}}, {{6, 3}, {3, 1}}};
+    const double *f = fit[dbl][el];
+    const bool halo = tr == 65;
+    const int owned = halo ? 64 : tr - 1, nt = halo ? 64 * tc + 64 : tr * tc;
+    const int per_cu = resident[dbl][el][nt > 256];
+    const double nb = (double)((op.ny + owned - 1) / owned) * ((op.nx + tc - 2) / (tc - 1)) * ((op.nz + lz - 1) / lz);
+    auto step = [&](double on_cu) { return f[2] + std::max(f[0], on_cu * nt * f[1]); };
+    const double slots = 256.0 * per_cu, full = floor(nb / slots), rest = nb - full * slots;
+    const double steps = std::min(lz, op.nz) + 2;
+    const double chain = full * step(per_cu) + (rest > 0 ? step(ceil(rest / 256.0)) : 0.0);
+    const double vb = sizeof(T) * (el ? 3 : 1);
+    const double loaded = nb * (tc + 1) * ((owned + 2) + 128.0 / vb) * steps * 1e-6;
+    return chain * steps + f[3] * loaded;
+}
+
+template <typename T>
+WalshTiles walsh_tile_rule(const OpDesc &op, int lean)
+{
+    static const int shapes[][2] = {{32, 8}, {16, 16}, {64, 4}, {64, 8}, {65, 7}};
+    WalshTiles best = {32, 8, 16};
+    double least = 1e300;
+    for (const auto &sh : shapes) {
+        if (lean && sh[0] != 32) continue;
+        // (16-row FP32 columns are 204-byte runs: the fit prefers them at
+        // 160^3, where they measured 11 % slower than 64x8)
+        if (sh[0] == 16 && sizeof(T) == 4) continue;
+        for (int lz = 1; lz <= 32; lz *= 2) {
+            const double c = tile_cost<T>(op, sh[0], sh[1], lz);
+            if (c < least) {
+                least = c;
+                best = {sh[0], sh[1], lz};
+            }
+        }
+    }
+    return best;
+}
+template WalshTiles walsh_tile_rule<float>(const OpDesc &, int);
+template WalshTiles walsh_tile_rule<double>(const OpDesc &, int);
 
 bool apply_dir_ok(const OpDesc &op)
 {

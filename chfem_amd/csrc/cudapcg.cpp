@@ -1267,7 +1267,8 @@ static int ensure_dinv()
     }
     if (g->precond) launch_jacobi<double>(g->dm.op64, g->dinv64, g->stream);
     else launch_fill<double>(g->dinv64, 1.0, n, g->stream);
-    if (g->precision == CHFEM_PREC_MIXED) launch_convert<double, float>(g->dinv64, g->dinv32, n, g->stream);
+    // (the memory-lean solvers hold no FP32 vectors)
+    if (g->dinv32) launch_convert<double, float>(g->dinv64, g->dinv32, n, g->stream);
     g->dinv_valid = true;
     return 1;
 }

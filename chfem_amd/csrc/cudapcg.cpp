@@ -78,6 +78,14 @@ struct Solver {
     double *lamu64 = nullptr;
     float *lamu32 = nullptr;
     bool walsh_ok = false;
+    // element-by-element strategy on the Walsh-basis operator: packed node
+    // keys built from the element map (N entries, valid until the map
+    // changes); with a scalar density field the inverse diagonal per node
+    uint16_t *ekeys = nullptr;
+    size_t ekeys_n = 0;
+    bool ekeys_valid = false;
+    double *dnode64 = nullptr;
+    float *dnode32 = nullptr;
     // per-node fluid keys for the Walsh-basis Stokes operator (N bytes)
     uint8_t *fkeys = nullptr;
     size_t fkeys_n = 0;
@@ -276,6 +284,7 @@ static cudapcgFlag_t free_solver_arrays()
     dfree(g->d64); dfree(g->q64); dfree(g->s64); dfree(g->dinv64);
     dfree(g->x32); dfree(g->r32); dfree(g->d32); dfree(g->q32); dfree(g->s32); dfree(g->dinv32);
     dfree(g->z2_64); dfree(g->q2_64); dfree(g->z2_32); dfree(g->q2_32);
+    dfree(g->dnode64); dfree(g->dnode32);
     dfree(g->xr64); dfree(g->hist);
     g->xr_n = g->hist_n = 0;
     for (int k = 0; k < RING_MAX; k++) { dfree(g->ring64[k]); dfree(g->ring32[k]); }
@@ -335,6 +344,7 @@ static cudapcgFlag_t alloc_solver_arrays()
 
 // Build the operator descriptors from the model and the local matrices.
 static bool is_lean();
+static bool is_minres();
 static int make_ops()
 {
     cudapcgModel_t *m = g->model;
@@ -395,13 +405,37 @@ static int make_ops()
         o.sdf.d = m->parametric_density_field;
         o.sdf.fmin = m->limits_density_field[0];
         o.sdf.fmax = m->limits_density_field[1];
-        use_walsh = false;  // the Walsh operator has no per-element scale
     }
+    // Element-by-element strategy: where the Walsh-basis operator takes the
+    // local matrices it computes the same product with a sixth of the
+    // matrix-core kernel's operations and the single-kernel iterations come
+    // with it (CHFEM_EBE or CHFEM_EBE_TILE set: the element kernels).
+    // Without a density field the element map is packed into node keys and
+    // the model runs as a node-by-node one.
+    const char *esel = getenv("CHFEM_EBE");
+    const bool ebe_kernels = esel || getenv("CHFEM_EBE_TILE");
+    o.ebe_matrix = o.ebe && ebe_kernels;
+    if (o.ebe && use_walsh && !ebe_kernels && !o.sdf.d && g->kinv64) {
+        if (g->ekeys_n != (size_t)o.N) {
+            dfree(g->ekeys);
+            g->ekeys_n = 0;
+            g->ekeys_valid = false;
+            if (hipMalloc(&g->ekeys, o.N * sizeof(uint16_t)) == hipSuccess) g->ekeys_n = o.N;
+            else (void)hipGetLastError();  // no room: the element kernels
+        }
+        if (g->ekeys_n) {
+            if (!g->ekeys_valid) launch_keys_from_elements(m->image, g->ekeys, o.ny, o.nx, o.nz, g->stream);
+            g->ekeys_valid = true;
+            o.ebe = 0;
+            o.keys = g->ekeys;
+        }
+    }
+    if (o.sdf.d && ebe_kernels) use_walsh = false;
+    if (o.ebe && !o.sdf.d) o.ebe_matrix = 1;
     const char *vsel = getenv("CHFEM_VECTOR");
     const bool kj = g->kinv64 && g->precond && !o.ebe && o.physics != PHY_FLUID && !(vsel && !strcmp(vsel, "stored"));
     o.kinv = nullptr;
     o.nmat = (int)g->dm.nmat;
-    const char *esel = getenv("CHFEM_EBE");
     o.ebe_atomic = (esel && !strcmp(esel, "atomic")) || o.physics == PHY_FLUID;
     o.ebe_tiles16 = esel && !strcmp(esel, "mfma16");
     g->dm.op64 = o;
@@ -412,6 +446,17 @@ static int make_ops()
     g->dm.op32.K = g->dm.K32;
     g->dm.op32.lamu = use_walsh ? g->lamu32 : nullptr;
     g->dm.op32.kinv = kj ? g->kinv32 : nullptr;
+    // density field: the single-kernel iterations read the inverse diagonal
+    // per node (filled with the stored diagonal, ensure_dinv)
+    g->dm.op64.dnode = g->dm.op32.dnode = nullptr;
+    if (o.sdf.d && use_walsh && !is_lean() && !is_minres() && g->arrays && !(vsel && !strcmp(vsel, "stored"))) {
+        if (!g->dnode64 && hipMalloc(&g->dnode64, o.N * sizeof(double)) == hipSuccess) g->dinv_valid = false;
+        if (g->precision == CHFEM_PREC_MIXED && !g->dnode32 && hipMalloc(&g->dnode32, o.N * sizeof(float)) == hipSuccess)
+            g->dinv_valid = false;
+        (void)hipGetLastError();  // no room: the loops with the stored diagonal
+        g->dm.op64.dnode = g->dnode64;
+        g->dm.op32.dnode = g->dnode32;
+    }
     if (!fixed_tile && !g->tuned && use_walsh) {
         const WalshTiles t64 = walsh_tile_rule<double>(o, is_lean()), t32 = walsh_tile_rule<float>(o, is_lean());
         g->dm.op64.tile_tr = t64.TR; g->dm.op64.tile_tc = t64.TC; g->dm.op64.tile_lz = t64.LZ;
@@ -624,7 +669,9 @@ static int run_pcg(const OpDesc &op, T *x, T *r, T *d, T *q, const T *dinv, bool
     const size_t n = op.ndof;
     hipStream_t st = g->stream;
     const bool kj = op.kinv != nullptr;
-    const bool fused = kj && d2 && fuse_dir_enabled() && apply_dir_ok(op);
+    // (with a density field only the single-kernel form: no key has the
+    // diagonal its update kernel would look up)
+    const bool fused = d2 && fuse_dir_enabled() && apply_dir_ok(op) && (kj || loop_mode<T>() == 2);
     const Ring<T> ring = fused ? dir_ring<T>(d, d2) : Ring<T>{};
     const unsigned W = fused ? (unsigned)ring.w : 1u;
     auto slot = [&](unsigned j) { return (T *)ring.p[j % W]; };
@@ -678,7 +725,8 @@ static int run_pcg(const OpDesc &op, T *x, T *r, T *d, T *q, const T *dinv, bool
     Reduce ra = make_guarded(FIN_ALPHA, 0), rdl = make_guarded(FIN_DELTA, 0), rc = make_guarded(FIN_CG1, 0);
     if (fused) {
         Reduce rz = make_reduce(FIN_STORE, S_TMP0);
-        launch_kj_to_z<T>(op, r, &rz, st);
+        if (kj) launch_kj_to_z<T>(op, r, &rz, st);
+        else launch_precond<T>(dinv, r, r, n, nullptr, st);
     }
     if (!arm_guard(tol * tol * fabs(delta0))) return -1;
     it = 0;
@@ -1269,6 +1317,9 @@ static int ensure_dinv()
     else launch_fill<double>(g->dinv64, 1.0, n, g->stream);
     // (the memory-lean solvers hold no FP32 vectors)
     if (g->dinv32) launch_convert<double, float>(g->dinv64, g->dinv32, n, g->stream);
+    const int nd = g->dm.op64.physics == PHY_ELASTIC ? 3 : 1;
+    if (g->dnode64) launch_node_jacobi<double>(g->dinv64, g->dnode64, nd, g->dm.op64.N, g->stream);
+    if (g->dnode32 && g->dinv32) launch_node_jacobi<float>(g->dinv32, g->dnode32, nd, g->dm.op64.N, g->stream);
     g->dinv_valid = true;
     return 1;
 }
@@ -1307,7 +1358,7 @@ static int run_mixed_reliable(bool x0set, unsigned &it_total, unsigned &sweeps, 
     // whole solve, the direction is kept across replacements) writes ring
     // slot j % w, and x += alpha_j d_j is applied per window of w iterations
     // and at each segment end
-    const bool fused = kj && g->s32 && fuse_dir_enabled() && apply_dir_ok(o32);
+    const bool fused = g->s32 && fuse_dir_enabled() && apply_dir_ok(o32) && (kj || loop_mode<float>() == 2);
     const Ring<float> ring = fused ? dir_ring<float>(d, g->s32) : Ring<float>{};
     const unsigned W = fused ? (unsigned)ring.w : 1u;
     auto slot = [&](unsigned j) { return (float *)ring.p[j % W]; };
@@ -1351,8 +1402,11 @@ static int run_mixed_reliable(bool x0set, unsigned &it_total, unsigned &sweeps, 
     // FP32 start: r = (float) r64, x = 0, d = M^-1 r, S[delta] = r.d
     launch_convert<double, float>(g->r64, r, n, st);
     launch_fill<float>(x, 0.0, n, st);
-    if (fused) launch_kj_to_z<float>(o32, r, &rd, st);
-    else if (kj) launch_kj_precond<float>(o32, r, d, &rd, st);
+    if (fused && kj) launch_kj_to_z<float>(o32, r, &rd, st);
+    else if (fused) {
+        launch_precond<float>(dinv, r, d, n, &rd, st);  // S[delta]; the loop's d is written by its first iteration
+        launch_precond<float>(dinv, r, r, n, nullptr, st);
+    } else if (kj) launch_kj_precond<float>(o32, r, d, &rd, st);
     else launch_precond<float>(dinv, r, d, n, &rd, st);
     // FP32 iterations are queued cg_batch() at a time; the device stops the
     // queue once r.z falls to the next replacement threshold
@@ -1433,7 +1487,8 @@ static int run_mixed_reliable(bool x0set, unsigned &it_total, unsigned &sweeps, 
         delta_rel = delta;
         float *rs = cg1 ? zb[(it_total + 1) & 1] : r;  // the next segment's first z
         launch_convert<double, float>(g->r64, rs, n, st);
-        if (fused) launch_kj_to_z<float>(o32, rs, &rz, st);
+        if (fused && kj) launch_kj_to_z<float>(o32, rs, &rz, st);
+        else if (fused) launch_precond<float>(dinv, rs, rs, n, nullptr, st);
         else if (!kj) launch_precond<float>(dinv, r, q, n, nullptr, st);  // stored-dinv direction reads z from q
         base = it_total;
         if (!arm_guard(thresh())) return -1;
@@ -1700,6 +1755,8 @@ cudapcgFlag_t cudapcgEnd(void)
     dfree(g->lamu32);
     dfree(g->fkeys);
     g->fkeys_n = 0;
+    dfree(g->ekeys);
+    g->ekeys_n = 0;
     dfree(g->kinv64);
     dfree(g->kinv32);
     dfree(g->btab64);
@@ -1767,6 +1824,7 @@ static cudapcgFlag_t alloc_model_device()
     const size_t n = m->nvars;
     dfree(g->r64);
     free_solver_arrays();
+    g->ekeys_valid = false;
     CHECK_HIP(hipMalloc(&g->r64, n * sizeof(double)));
     if (g->analysis_flag != CUDAPCG_FLUID_3D) {
         if (!m->image) CHECK_HIP(hipMalloc(&m->image, sizeof(cudapcgMap_t) * m->nelem));
@@ -1871,6 +1929,7 @@ cudapcgFlag_t cudapcgSetX0(cudapcgVar_t *x0, cudapcgFlag_t mustInterpolate)
 cudapcgFlag_t cudapcgSetImage(cudapcgMap_t *img)
 {
     if (!g || !g->model || !img || !g->model->image) return CUDAPCG_FALSE;
+    g->ekeys_valid = false;
     CHECK_HIP(hipMemcpyAsync(g->model->image, img, g->model->nelem * sizeof(cudapcgMap_t), hipMemcpyHostToDevice,
                              g->stream));
     CHECK_HIP(hipStreamSynchronize(g->stream));
@@ -2160,6 +2219,7 @@ double cudapcgOperatorBench(cudapcgFlag_t precision, unsigned int reps, cudapcgF
     if (dir) {
         // CG-loop form: r = x, directions alternate between d and s
         if (!g->precond || !apply_dir_ok(precision == CHFEM_PREC_MIXED ? g->dm.op32 : g->dm.op64)) return -1.0;
+        if (!cg1 && g->dm.op64.sdf.d) return -1.0;  // single-kernel form only
         if (!set_scalar(S_DELTA_OLD, 1.0) || !set_scalar(S_DELTA, 0.5) || !set_scalar(S_ALPHA, 0.0) ||
             !set_scalar(S_BPREV, 0.5))
             return -1.0;

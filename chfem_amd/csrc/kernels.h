@@ -95,9 +95,18 @@ struct OpDesc {
     // (thermal/elastic NBN)
     const void *kinv;
     int nmat;
-    // EBE: 1 selects the reference-style element kernel with atomics instead
-    // of the matrix-core kernel (ebe_mfma.hip; up to 4 materials)
+    // inverse Jacobi diagonal per node (N entries, precision of K) of a model
+    // with a scalar density field on the Walsh-basis operator: selects its
+    // single-kernel CG form
+    const void *dnode;
+    // EBE with local matrices that the Walsh-basis operator does not take (or
+    // CHFEM_EBE / CHFEM_EBE_TILE set): 1 selects the reference-style element
+    // kernel with atomics instead of the matrix-core kernel (ebe_mfma.hip; up
+    // to 4 materials)
     int ebe_atomic;
+    // EBE: 1 keeps the matrix-core kernel where lamu would allow the
+    // Walsh-basis operator
+    int ebe_matrix;
     // EBE matrix-core kernel in FP32: 1 selects the 16x16x4 column-tile form
     // (the FP64 form) instead of the 4x4x1 block form
     int ebe_tiles16;
@@ -186,6 +195,11 @@ template <typename T> void launch_ebe_mfma(const OpDesc &op, const T *v, T *q, c
 // red.partials (fixed order) and publishes them as red.fin says.  Every
 // launcher that takes a Reduce calls it after its kernel.
 void launch_reduce_finish(const Reduce &red, unsigned nb, int nv, hipStream_t s);
+
+// packed NBN keys of an element material map (2 bits per element around the
+// node), and dnode[i] = dinv[nd * i]
+void launch_keys_from_elements(const uint16_t *elems, uint16_t *keys, int ny, int nx, int nz, hipStream_t s);
+template <typename T> void launch_node_jacobi(const T *dinv, T *dnode, int nd, uint32_t N, hipStream_t s);
 
 // dinv[i] = 1 / diag(A)_i in precision T, from the keys (thermal/elastic) or the
 // Stokes pore/border structure.

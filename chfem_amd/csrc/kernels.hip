@@ -1240,12 +1240,16 @@ void launch_apply(const OpDesc &op, const T *v, T *q, const Reduce *red, hipStre
         else k_fluid<T, false><<<grid_for(nt), BS, 0, s>>>(v, q, op.dof2node, op.node2dof, op.bkeys, K, op.ny, op.nx, op.nz, op.nvel, op.nborder, rr);
         return;
     }
-    if (op.ebe && op.nmat <= 4 && !op.ebe_atomic) {
+    if (op.ebe && op.nmat <= 4 && !op.ebe_atomic && (op.ebe_matrix || !op.lamu)) {
         launch_ebe_mfma<T>(op, v, q, red, s);
         return;
     }
     if (op.lamu) {
-        // Walsh-basis elastic (isotropic) or conduction operator, NBN or EBE
+        // Walsh-basis elastic (isotropic) or conduction operator, NBN or EBE,
+        // with or without a density field.  The matrix-core kernel does 6
+        // times its operations for the same product: at 96^3 two-phase FP64
+        // elastic it took 159 us per apply, this one with the whole CG
+        // iteration inside about 42 us
         WalshTiles t = {op.tile_tr, op.tile_tc, op.tile_lz};
         launch_walsh<T>(op, (const T *)op.lamu, v, q, red, t, s);
         return;
@@ -1265,6 +1269,48 @@ void launch_apply(const OpDesc &op, const T *v, T *q, const Reduce *red, hipStre
         else k_elastic_nbn<T, false><<<grid_for(op.N), BS, 0, s>>>(v, q, op.keys, K, op.ny, op.nx, op.nz, op.N, rr);
     }
 }
+
+// One work-item per node, the 8 element reads of a wavefront in 4 column runs
+// of two layers (cached): bound by its 4 B per node.
+__global__ void __launch_bounds__(BS) k_keys_from_elements(const uint16_t *__restrict__ elems,
+                                                           uint16_t *__restrict__ keys, int ny, int nx, int nz,
+                                                           uint32_t N)
+{
+    for (uint32_t i = blockIdx.x * BS + threadIdx.x; i < N; i += gridDim.x * BS) {
+        int r, c, l;
+        node_rcl(i, ny, nx, r, c, l);
+        const Nbh h = make_nbh(r, c, l, ny, nx, nz);
+        unsigned key = 0;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            // element (r - DR, c - DC, l - DL) has this node as its local node e
+            const size_t el = h.lo[1 - LDL(e)] + h.co[1 - LDC(e)] + h.ro[1 - LDR(e)];
+            key |= ((unsigned)elems[el] & 3u) << (2 * e);
+        }
+        keys[i] = (uint16_t)key;
+    }
+}
+
+void launch_keys_from_elements(const uint16_t *elems, uint16_t *keys, int ny, int nx, int nz, hipStream_t s)
+{
+    const uint32_t N = (uint32_t)((size_t)ny * nx * nz);
+    k_keys_from_elements<<<grid_for(N), BS, 0, s>>>(elems, keys, ny, nx, nz, N);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(BS) k_node_jacobi(const T *__restrict__ dinv, T *__restrict__ dnode, int nd,
+                                                    uint32_t N)
+{
+    for (uint32_t i = blockIdx.x * BS + threadIdx.x; i < N; i += gridDim.x * BS) dnode[i] = dinv[(size_t)nd * i];
+}
+
+template <typename T>
+void launch_node_jacobi(const T *dinv, T *dnode, int nd, uint32_t N, hipStream_t s)
+{
+    k_node_jacobi<T><<<grid_for(N), BS, 0, s>>>(dinv, dnode, nd, N);
+}
+template void launch_node_jacobi<float>(const float *, float *, int, uint32_t, hipStream_t);
+template void launch_node_jacobi<double>(const double *, double *, int, uint32_t, hipStream_t);
 
 template <typename T>
 void launch_jacobi(const OpDesc &op, T *dinv, hipStream_t s)

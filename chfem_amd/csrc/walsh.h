@@ -245,6 +245,12 @@ struct DirFuse {
     // M^-1 A v in place in q (z) with z.diag z; M^-1 from kinv by the owned
     // node's packed key (kinv == nullptr: no preconditioner)
     int lean;
+    // scalar density field (SDF kernels): the element scale, and for the
+    // single-kernel CG the inverse Jacobi diagonal per node (with a density
+    // it is no function of the key; the diagonal of an isotropic element is
+    // the same for the three components, so one value serves a node)
+    Sdf sdf;
+    const T *dnode;
 };
 
 // Sums a tile contributes to the launch's reductions: d.q, and for the
@@ -277,7 +283,9 @@ struct TileSums {
 // one to one, the batched solver (batch.hip) through a tile table.  FUSE: the
 // input is the fused direction update of DirFuse (the dot is then d.q with
 // the updated d).
-template <typename T, int ND, int TR, int TC, bool DOT, int FM = 0, bool HALO = false>
+// SDF: every element's material coefficients are scaled by its density (one
+// uint16 per element, read with the material; 7 multiplies per element).
+template <typename T, int ND, int TR, int TC, bool DOT, int FM = 0, bool HALO = false, bool SDF = false>
 __device__ __forceinline__ TileSums walsh_tile(const T *__restrict__ v, T *__restrict__ q,
                                                const uint16_t *__restrict__ keys, const T *__restrict__ lamu, int ebe,
                                                int ny, int nx, int nz, int LZ, int bx, int by, int bz,
@@ -399,6 +407,11 @@ __device__ __forceinline__ TileSums walsh_tile(const T *__restrict__ v, T *__res
                                   : 0u;
     // (mat_key takes the wrapped layer index)
     auto mat_key = [&](int lw) -> uint16_t { return (keys + (size_t)lw * nxy)[eoff]; };
+    // SDF: the element's density value, read with its material
+    auto dens_key = [&](int lw) -> uint16_t { return SDF ? (fz.sdf.d + (size_t)lw * nxy)[eoff] : (uint16_t)0; };
+    auto dens_scale = [&](uint32_t d) -> T {
+        return SDF ? (T)((double)d * (1.0 / 65535.0) * (fz.sdf.fmax - fz.sdf.fmin) + fz.sdf.fmin) : T(1);
+    };
     auto material = [&](uint32_t kv) -> int {
         // NBN keys: node (r,c,l) is local node 3 of element (r,c,l); EBE: element map
         if (!elem_ok) return 4;
@@ -417,8 +430,15 @@ __device__ __forceinline__ TileSums walsh_tile(const T *__restrict__ v, T *__res
     // (work-items without an element read in-tile LDS entries, all written
     // each step from finite vector values, and evaluate them with the zero
     // material 4)
-    auto element = [&](const T *cur, const T *nxt, int m, T (&A)[ND], T (&Af)[ND]) {
+    auto element = [&](const T *cur, const T *nxt, int m, T sc, T (&A)[ND], T (&Af)[ND]) {
         T f[8][ND];
+        T cs[WCOEF];
+        const T *coef = smat + WCOEF * m;
+        if constexpr (SDF) {
+#pragma unroll
+            for (int i = 0; i < (ND == 3 ? 7 : 3); i++) cs[i] = coef[i] * sc;
+            coef = cs;
+        }
         T u[8][ND];
 #pragma unroll
         for (int k = 0; k < 8; k++) {
@@ -428,12 +448,12 @@ __device__ __forceinline__ TileSums walsh_tile(const T *__restrict__ v, T *__res
             for (int a = 0; a < ND; a++) u[k][a] = src[o + a];
         }
         if constexpr (ND == 3) {
-            element_forces(u, smat + WCOEF * m, f);
+            element_forces(u, coef, f);
         } else {
             T u1[8], f1[8];
 #pragma unroll
             for (int k = 0; k < 8; k++) u1[k] = u[k][0];
-            conduction_forces(u1, smat + WCOEF * m, f1);
+            conduction_forces(u1, coef, f1);
 #pragma unroll
             for (int k = 0; k < 8; k++) f[k][0] = f1[k];
         }
@@ -484,16 +504,18 @@ __device__ __forceinline__ TileSums walsh_tile(const T *__restrict__ v, T *__res
     const int lwm = wrapl(l0 - 1), lw0 = wrapl(l0);
     int lw1 = next_layer(lw0), lw2 = next_layer(lw1);  // wrapped l + 1, l + 2 of the step
     fetch(lwm);
-    uint16_t mk = mat_key(lwm);
+    uint16_t mk = mat_key(lwm), dk = dens_key(lwm);
     store(cur, zcur);
     fetch(lw0);
     store(nxt, znxt);
     int m = material(mk);
+    T sc = dens_scale(dk);
     mk = mat_key(lw0);
+    dk = dens_key(lw0);
     __syncthreads();
     fetch(lw1);
     T A[ND], Af[ND];
-    element(cur, nxt, m, A, Af);
+    element(cur, nxt, m, sc, A, Af);
     __syncthreads();
     T acc[ND];
     if (own) halo_row(A, Af);
@@ -501,6 +523,7 @@ __device__ __forceinline__ TileSums walsh_tile(const T *__restrict__ v, T *__res
     for (int a = 0; a < ND; a++) acc[a] = own ? Af[a] + bleft[ND + a] : T(0);
     store(cur, zcur);  // layer l0 + 1 replaces layer l0 - 1
     m = material(mk);
+    sc = dens_scale(dk);
     uint32_t kraw = mk;  // packed key of the owned node at the current layer (CG1 dinv)
     {
         T *t = cur; cur = nxt; nxt = t;  // cur = layer l0, nxt = layer l0 + 1
@@ -522,6 +545,7 @@ __device__ __forceinline__ TileSums walsh_tile(const T *__restrict__ v, T *__res
         // and none is pending across the loop's back edge.
         const uint32_t kcur = kraw;
         mk = mat_key(lw1);
+        dk = dens_key(lw1);
         // CG1: dinv and diag of the owned node (its key is the element's,
         // loaded a step ahead), read after this layer's elements
         T mo[CG1 || LEAN ? ND : 1], dgo[CG1 || LEAN ? ND : 1];
@@ -553,7 +577,7 @@ __device__ __forceinline__ TileSums walsh_tile(const T *__restrict__ v, T *__res
         fetch(lw2);
         lw1 = lw2;
         lw2 = next_layer(lw2);
-        element(cur, nxt, m, A, Af);
+        element(cur, nxt, m, sc, A, Af);
         __syncthreads();
         // the prefetched plane goes to LDS before this layer's node results
         // are stored, so waiting for the loads does not wait for the stores
@@ -565,10 +589,21 @@ __device__ __forceinline__ TileSums walsh_tile(const T *__restrict__ v, T *__res
         m = material(mk);
         kraw = mk;
         pin_here(m);
+        if constexpr (SDF) {
+            asm volatile("" : "+v"(dk));
+            sc = dens_scale(dk);
+        }
         // (loaded here rather than before the elements: six fewer registers
         // live across them, 3 % faster at 256^3; the table rows of the few
         // keys in use stay in the caches)
-        if constexpr (CG1) {
+        if constexpr (CG1 && SDF) {
+            const T di = fz.dnode[(size_t)l * nxy + own_off], dg = T(1) / di;
+#pragma unroll
+            for (int a = 0; a < ND; a++) {
+                mo[a] = di;
+                dgo[a] = dg;
+            }
+        } else if constexpr (CG1) {
 #pragma unroll
             for (int a = 0; a < ND; a++) {
                 mo[a] = fz.kinv[ND * kcur + a];

@@ -10,10 +10,10 @@
 
 namespace chfem {
 
-template <typename T, int ND, int TR, int TC, bool DOT, int FM, bool HALO>
-__global__ void __launch_bounds__(TR *TC + (HALO ? 64 : 0)) k_walsh(const T *__restrict__ v, T *__restrict__ q,
-                                                   const uint16_t *__restrict__ keys, const T *__restrict__ lamu,
-                                                   int ebe, int ny, int nx, int nz, int LZ, Reduce red, DirFuse<T> fz)
+template <typename T, int ND, int TR, int TC, bool DOT, int FM, bool HALO, bool SDF>
+__device__ __forceinline__ void walsh_block(const T *__restrict__ v, T *__restrict__ q,
+                                            const uint16_t *__restrict__ keys, const T *__restrict__ lamu, int ebe,
+                                            int ny, int nx, int nz, int LZ, const Reduce &red, DirFuse<T> fz)
 {
     constexpr bool FUSE = FM == 1 || FM == 2;
     if (DOT && stopped(red)) return;
@@ -41,8 +41,9 @@ __global__ void __launch_bounds__(TR *TC + (HALO ? 64 : 0)) k_walsh(const T *__r
     unsigned k = b / 8u;
     if (FM == 2 && DOT && red.guard && (((unsigned)red.S[S_ITER]) & 1u)) k = (xcd < rem ? per + 1u : per) - 1u - k;
     const unsigned t = (xcd < rem ? xcd * (per + 1u) : rem * (per + 1u) + (xcd - rem) * per) + k;
-    const TileSums ts = walsh_tile<T, ND, TR, TC, DOT, FM, HALO>(v, q, keys, lamu, ebe, ny, nx, nz, LZ, (int)(t % gx),
-                                                           (int)((t / gx) % gy), (int)(t / (gx * gy)), fz);
+    const TileSums ts = walsh_tile<T, ND, TR, TC, DOT, FM, HALO, SDF>(v, q, keys, lamu, ebe, ny, nx, nz, LZ,
+                                                                      (int)(t % gx), (int)((t / gx) % gy),
+                                                                      (int)(t / (gx * gy)), fz);
     if (DOT && FM == 2) {
         double vv[4] = {ts.dq, ts.zq, ts.qmq, ts.zdz};
         store_partials<4>(red, vv);
@@ -52,19 +53,39 @@ __global__ void __launch_bounds__(TR *TC + (HALO ? 64 : 0)) k_walsh(const T *__r
     }
 }
 
+template <typename T, int ND, int TR, int TC, bool DOT, int FM, bool HALO>
+__global__ void __launch_bounds__(TR *TC + (HALO ? 64 : 0)) k_walsh(const T *__restrict__ v, T *__restrict__ q,
+                                                   const uint16_t *__restrict__ keys, const T *__restrict__ lamu,
+                                                   int ebe, int ny, int nx, int nz, int LZ, Reduce red, DirFuse<T> fz)
+{
+    walsh_block<T, ND, TR, TC, DOT, FM, HALO, false>(v, q, keys, lamu, ebe, ny, nx, nz, LZ, red, fz);
+}
+
+// with a scalar density field (op.sdf): 32x8 tiles, and the 65x7 ones where
+// the rule prefers long rows
+template <typename T, int ND, int TR, int TC, bool DOT, int FM, bool HALO>
+__global__ void __launch_bounds__(TR *TC + (HALO ? 64 : 0)) k_walsh_sdf(const T *__restrict__ v, T *__restrict__ q,
+                                                   const uint16_t *__restrict__ elems, const T *__restrict__ lamu,
+                                                   int ny, int nx, int nz, int LZ, Reduce red, DirFuse<T> fz)
+{
+    walsh_block<T, ND, TR, TC, DOT, FM, HALO, true>(v, q, elems, lamu, 1, ny, nx, nz, LZ, red, fz);
+}
+
 template <typename T, int ND>
 static void launch_walsh_nd(const OpDesc &op, const T *lamu, const T *v, T *q, const Reduce *red, WalshTiles t,
                             hipStream_t s, const DirFuse<T> *fz, const hipEvent_t *ev)
 {
     Reduce rr = {nullptr, nullptr, 0, 0, 0};
     if (red) rr = *red;
-    DirFuse<T> f = {nullptr, nullptr, T(0), T(0), 1, 0, nullptr, nullptr, nullptr, 0, T(0), 0};
+    DirFuse<T> f = {nullptr, nullptr, T(0), T(0), 1, 0, nullptr, nullptr, nullptr, 0, T(0), 0, {}, nullptr};
     if (fz) f = *fz;
+    f.sdf = op.sdf;
+    f.dnode = (const T *)op.dnode;
     // lean forms of the memory-lean solvers: one tile shape (32 x 8)
     const bool lean = fz && fz->lean;
     // single-kernel CG form: the dinv table given (only launch_apply_cg1
     // sets it; its z output may be absent)
-    const bool cg1 = fz && fz->kinv;
+    const bool cg1 = fz && (fz->kinv || (op.sdf.d && fz->dnew));
     int LZ = t.LZ > 0 ? t.LZ : 16;
     {
         // keep the block count within the reduction partials buffer
@@ -117,6 +138,33 @@ static void launch_walsh_nd(const OpDesc &op, const T *lamu, const T *v, T *q, c
         WALSH_LAUNCH_LEAN(32, 8)
 #undef WALSH_LAUNCH_LEAN
     }
+    if (op.sdf.d) {
+#define WALSH_GO_SDF(TRv, TCv, H, DOTv, FMv)                                                            \
+    if (ev) hipExtLaunchKernelGGL(k_walsh_sdf<T, ND, TRv, TCv, DOTv, FMv, H>, dim3(grid), dim3(nt), 0, s, ev[0], \
+                                  ev[1], 0, v, q, op.keys, lamu, op.ny, op.nx, op.nz, LZ, rr, f);       \
+    else k_walsh_sdf<T, ND, TRv, TCv, DOTv, FMv, H><<<grid, nt, 0, s>>>(v, q, op.keys, lamu, op.ny, op.nx, op.nz, \
+                                                                        LZ, rr, f);
+#define WALSH_LAUNCH_SDF(TRv, TCv, H)                                                                   \
+    {                                                                                                   \
+        constexpr int orows = H ? TRv : TRv - 1, nt = TRv * TCv + (H ? 64 : 0);                         \
+        const unsigned grid = (unsigned)((op.ny + orows - 1) / orows) * ((op.nx + TCv - 2) / (TCv - 1)) * \
+                              ((op.nz + LZ - 1) / LZ);                                                  \
+        if (cg1) {                                                                                      \
+            WALSH_GO_SDF(TRv, TCv, H, true, 2)                                                          \
+            launch_reduce_finish(rr, grid, 4, s);                                                       \
+        } else if (red) {                                                                               \
+            WALSH_GO_SDF(TRv, TCv, H, true, 0)                                                          \
+            launch_reduce_finish(rr, grid, 1, s);                                                       \
+        } else {                                                                                        \
+            WALSH_GO_SDF(TRv, TCv, H, false, 0)                                                         \
+        }                                                                                               \
+        return;                                                                                         \
+    }
+        if (t.TR == 65) WALSH_LAUNCH_SDF(64, 7, true)
+        WALSH_LAUNCH_SDF(32, 8, false)
+#undef WALSH_LAUNCH_SDF
+#undef WALSH_GO_SDF
+    }
     if constexpr (sizeof(T) == 4) {
         if (t.TR == 65 && t.TC == 15) WALSH_LAUNCH(64, 15, true)
     }
@@ -142,7 +190,7 @@ template <typename T>
 void launch_walsh_lean(const OpDesc &op, int form, const T *v, T *z, const void *kinv, const Reduce *red,
                        hipStream_t s)
 {
-    DirFuse<T> f = {nullptr, nullptr, T(0), T(0), 1, 0, nullptr, nullptr, (const T *)kinv, 0, T(0), form};
+    DirFuse<T> f = {nullptr, nullptr, T(0), T(0), 1, 0, nullptr, nullptr, (const T *)kinv, 0, T(0), form, {}, nullptr};
     const WalshTiles t = {32, 8, op.tile_lz};
     launch_walsh<T>(op, (const T *)op.lamu, v, z, red, t, s, &f, nullptr);
 }
@@ -199,6 +247,7 @@ WalshTiles walsh_tile_rule(const OpDesc &op, int lean)
     double least = 1e300;
     for (const auto &sh : shapes) {
         if (lean && sh[0] != 32) continue;
+        if (op.sdf.d && sh[0] != 32 && sh[0] != 65) continue;
         // (16-row FP32 columns are 204-byte runs: the fit prefers them at
         // 160^3, where they measured 11 % slower than 64x8)
         if (sh[0] == 16 && sizeof(T) == 4) continue;
@@ -218,14 +267,16 @@ template WalshTiles walsh_tile_rule<double>(const OpDesc &, int);
 bool apply_dir_ok(const OpDesc &op)
 {
     // the operators launch_apply sends to the Walsh kernel, with key-Jacobi on
-    return op.physics != PHY_FLUID && !op.ebe && op.lamu && op.kinv;
+    // or a stored one per node (scalar density field; single-kernel form only)
+    return op.physics != PHY_FLUID && op.lamu && (op.sdf.d ? op.dnode != nullptr : !op.ebe && op.kinv);
 }
 
 template <typename T>
 void launch_apply_dir(const OpDesc &op, const T *z, const T *dold, T *dnew, T *q, const Reduce *red, hipStream_t s,
                       const hipEvent_t *ev)
 {
-    const DirFuse<T> f = {z, dnew, T(0), T(0), dold ? 0 : 1, 0, nullptr, nullptr, nullptr, 0, T(0), 0};
+    const DirFuse<T> f = {z, dnew, T(0), T(0), dold ? 0 : 1, 0, nullptr, nullptr, nullptr, 0, T(0), 0, {},
+                          nullptr};
     const WalshTiles t = {op.tile_tr, op.tile_tc, op.tile_lz};
     launch_walsh<T>(op, (const T *)op.lamu, dold, q, red, t, s, &f, ev);
 }
@@ -239,7 +290,7 @@ void launch_apply_cg1(const OpDesc &op, const T *zold, const T *qold, const T *d
     // pending update)
     const int zr = dold2 && p ? 1 : 0;
     const DirFuse<T> f = {zr ? dold2 : zold, dnew, T(0), T(0), first, p, p ? qold : zold, znew, (const T *)op.kinv,
-                          zr, T(0), 0};
+                          zr, T(0), 0, {}, nullptr};
     const WalshTiles t = {op.tile_tr, op.tile_tc, op.tile_lz};
     launch_walsh<T>(op, (const T *)op.lamu, dold, qnew, red, t, s, &f, ev);
 }

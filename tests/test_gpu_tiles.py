@@ -42,3 +42,60 @@ def test_rule_tile_solves(shape, which, precision):
             assert abs(int(st.iterations) - itr) <= 2
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("env", [None, "mfma"], ids=["default", "matrix-cores"])
+@pytest.mark.parametrize("which", ["elastic", "thermal"])
+@pytest.mark.parametrize("shape", [(3, 2, 4), (9, 70, 40), (17, 33, 65)], ids=lambda s: "x".join(map(str, s)))
+def test_element_strategy(shape, which, env, monkeypatch):
+    """The element-by-element strategy on its default operator and on the
+    matrix-core kernel: apply to 1e-12, solves to the FP64 stop rule, then a
+    solve of another image set on the same solver (its node keys are
+    rebuilt)."""
+    if env:
+        monkeypatch.setenv("CHFEM_EBE", env)
+    rng = np.random.default_rng(sum(shape))
+    props = [1.0, 0.3, 10.0, 0.2, 4.0, 0.25] if which == "elastic" else [1.0, 10.0, 3.5]
+    images = [rng.choice(np.array([0, 100, 255], np.uint8), size=shape, p=[.5, .3, .2]) for _ in range(2)]
+    ms = [H.model(H.ELASTIC if which == "elastic" else H.THERMAL, i, props, colors=(0, 100, 255)) for i in images]
+    s = H.GpuSolver(ms[0], strategy=1, tol=1e-9)
+    try:
+        for m in ms:
+            elem = m.elem.copy()
+            assert s.L.cudapcgSetImage(s.ptr(elem)) == 1
+            v = rng.standard_normal(m.ndof)
+            assert rel(s.apply(v), m.apply(v, strategy=1)) < 1e-12
+            x, ok, st = s.solve(m.rhs(0))
+            xr, okr, itr, _ = m.solve(0, tol=1e-9, strategy=1)
+            assert ok and okr and abs(int(st.iterations) - itr) <= 2
+            assert rel(m.update_c(0, x), m.update_c(0, xr)) < 1e-7
+    finally:
+        s.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("solver", [0, 1, 2], ids=["cg", "minres", "cg3"])
+@pytest.mark.parametrize("which", ["elastic", "thermal"])
+@pytest.mark.parametrize("shape", [(3, 2, 4), (9, 70, 40), (24, 24, 24)], ids=lambda s: "x".join(map(str, s)))
+def test_density_solves(shape, which, solver, precision):
+    """Scalar density field (densities down to 1 % of the largest) with every
+    kind of loop, against the oracle's solve of the same scaled elements;
+    residual 1e-9 and a condition of the field below 1000 give 1e-6 in C."""
+    rng = np.random.default_rng(sum(shape) + solver)
+    img = rng.choice(np.array([0, 255], np.uint8), size=shape)
+    m = H.model(H.ELASTIC, img, [1.0, 0.3, 1.0, 0.2]) if which == "elastic" else H.model(H.THERMAL, img, [1.0, 2.0])
+    d = rng.integers(0, 65536, size=m.N).astype(np.uint16)
+    lo, hi = 0.01, 1.0
+    m.set_element_scale(d.astype(np.float64) * (1.0 / 65535.0) * (hi - lo) + lo)
+    s = H.GpuSolver(m, strategy=1, solver=solver, precision=precision, tol=1e-9)
+    try:
+        assert s.L.cudapcgSetParametricDensityField(s.ptr(d), lo, hi) == 1
+        v = rng.standard_normal(m.ndof) if solver < 2 else None
+        if v is not None:
+            assert rel(s.apply(v), m.apply(v, strategy=1)) < 1e-12
+        x, ok, st = s.solve(m.rhs(0))
+        xr, okr, itr, _ = m.solve(0, tol=1e-9, strategy=1)
+        assert ok and okr
+        assert rel(m.update_c(0, x), m.update_c(0, xr)) < 1e-6
+    finally:
+        s.close()

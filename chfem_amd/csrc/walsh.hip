@@ -16,7 +16,10 @@ __device__ __forceinline__ void walsh_block(const T *__restrict__ v, T *__restri
                                             int ny, int nx, int nz, int LZ, const Reduce &red, DirFuse<T> fz)
 {
     constexpr bool FUSE = FM == 1 || FM == 2;
-    if (DOT && stopped(red)) return;
+    // the scalars are read together, before the stop flag is tested: one
+    // read latency at the head of the launch instead of two
+    const double done = DOT && red.guard ? red.S[S_DONE] : 0.0;
+    double iter = 0.0;
     // beta of the fused direction update, as k_kj_pcg_dir forms it
     if (FUSE && !fz.first) fz.beta = (T)(red.S[S_DELTA] / red.S[S_DELTA_OLD]);
     // single-kernel CG: alpha of the previous iteration for the deferred z
@@ -27,6 +30,8 @@ __device__ __forceinline__ void walsh_block(const T *__restrict__ v, T *__restri
     if (FM == 2 && fz.zring) fz.bprev = (T)red.S[S_BPREV];
     // lean z update: alpha of this iteration
     if (FM == 3) fz.alpha = fz.lean == LEAN_ZUPD ? (T)red.S[S_ALPHA] : T(0);
+    if (FM == 2 && DOT && red.guard) iter = red.S[S_ITER];
+    if (done != 0.0) return;
     // 1-D grid; blocks are dispatched to the 8 XCDs round-robin (block b to
     // XCD b % 8), so each XCD is given one contiguous range of tiles (rows of
     // tiles fastest): tiles that share halo nodes then run on the same XCD at
@@ -39,7 +44,7 @@ __device__ __forceinline__ void walsh_block(const T *__restrict__ v, T *__restri
     const unsigned gx = (unsigned)(ny + OR - 1) / OR, gy = (unsigned)(nx + TC - 2) / (TC - 1);
     const unsigned b = blockIdx.x, nb = gridDim.x, per = nb / 8u, rem = nb % 8u, xcd = b % 8u;
     unsigned k = b / 8u;
-    if (FM == 2 && DOT && red.guard && (((unsigned)red.S[S_ITER]) & 1u)) k = (xcd < rem ? per + 1u : per) - 1u - k;
+    if (FM == 2 && DOT && red.guard && ((unsigned)iter & 1u)) k = (xcd < rem ? per + 1u : per) - 1u - k;
     const unsigned t = (xcd < rem ? xcd * (per + 1u) : rem * (per + 1u) + (xcd - rem) * per) + k;
     const TileSums ts = walsh_tile<T, ND, TR, TC, DOT, FM, HALO, SDF>(v, q, keys, lamu, ebe, ny, nx, nz, LZ,
                                                                       (int)(t % gx), (int)((t / gx) % gy),

@@ -150,6 +150,8 @@ Reduce make_reduce(int fin, int slot)
     r.fin = fin;
     r.slot = slot;
     r.guard = 0;
+    r.partials2 = nullptr;
+    r.nb2 = 0;
     return r;
 }
 
@@ -955,10 +957,30 @@ static int run_minres(const OpDesc &op, T *x, T *r, T *d, T *q, T *s, const T *d
     const unsigned W = rng ? (unsigned)ring.w : 1u;
     auto slot = [&](unsigned j) { return (T *)ring.p[j % W]; };
     unsigned issued = 1, flushed = 0;  // iterations queued, and folded into x
+    // Stokes: M^-1 by DOF class (the values of the stored diagonal) in the
+    // vector kernels, which then stream one vector less each
+    const FluidJac fj = {g->fl_vinv, g->fl_pinv, g->btab64, op.bkeys, op.nvel};
+    const FluidJac *cls = op.physics == PHY_FLUID && g->precond && g->btab64 && op.bkeys ? &fj : nullptr;
     launch_precond<T>(dinv, q, nullptr, n, &ra, st);
     it = 1;
-    launch_minres_update<T>(rng ? nullptr : x, r, d, q, dinv, &rs, n, st);
-    timed_apply<T>(op, r, s, &rdl);
+    // queued loops finish the update's residual sum together with the
+    // operator's r.Ar (one finishing block and its launch gap less per
+    // iteration; the operator launch then runs once more after the stop, its
+    // result unused): the update's partials lie behind the operator's
+    auto update_apply = [&](T *xu, const T *dj) {
+        if (!queued) {
+            launch_minres_update<T>(xu, r, dj, q, dinv, cls, &rs, n, st);
+            timed_apply<T>(op, r, s, &rdl);
+            return;
+        }
+        Reduce ru = rs, rsd = rdl;
+        ru.partials = g->partials + (size_t)MAX_PARTIAL_BLOCKS;
+        rsd.fin = FIN_STOP_DELTA;
+        rsd.partials2 = ru.partials;
+        rsd.nb2 = launch_minres_update<T>(xu, r, dj, q, dinv, cls, &ru, n, st, false);
+        timed_apply<T>(op, r, s, &rsd);
+    };
+    update_apply(rng ? nullptr : x, d);
     if (!sync_loop()) return -1;
     double stop = g->Sh[S_STOP], metric = 1.0;
     bool cont = above(stop, res0, tol);
@@ -973,18 +995,16 @@ static int run_minres(const OpDesc &op, T *x, T *r, T *d, T *q, T *s, const T *d
         for (unsigned b = 0; b < nb; b++) {
             if (rng) {
                 const unsigned j = issued;
-                launch_minres_dir<T>(slot(j - 1), slot(j), q, r, s, dinv, g->S, 0, &ra, n, st);
-                launch_minres_update<T>(nullptr, r, slot(j), q, dinv, &rs, n, st);
-                timed_apply<T>(op, r, s, &rdl);
+                launch_minres_dir<T>(slot(j - 1), slot(j), q, r, s, dinv, cls, g->S, 0, &ra, n, st);
+                update_apply(nullptr, slot(j));
                 issued = j + 1;
                 if (issued - flushed == W) {
                     launch_ring_flush<T>(x, ring, flushed, issued, 0, g->S, n, st);
                     flushed = issued;
                 }
             } else {
-                launch_minres_dir<T>(d, d, q, r, s, dinv, g->S, 0, &ra, n, st);
-                launch_minres_update<T>(x, r, d, q, dinv, &rs, n, st);
-                timed_apply<T>(op, r, s, &rdl);
+                launch_minres_dir<T>(d, d, q, r, s, dinv, cls, g->S, 0, &ra, n, st);
+                update_apply(x, d);
             }
         }
         if (!sync_loop()) return -1;

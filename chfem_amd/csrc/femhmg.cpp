@@ -1432,6 +1432,8 @@ logical hmgUpdateCNoAlloc(unsigned int dir, const double *x_dev, double *Ccol_de
     red.fin = FIN_STORE;
     red.slot = 0;
     red.guard = 0;
+    red.partials2 = nullptr;
+    red.nb2 = 0;
     hipStream_t st = active_stream();
     if (m.analysis == HMG_FLUID) {
         launch_fluid_velocity_sum<double>(dm->op64, x_dev, &red, st);

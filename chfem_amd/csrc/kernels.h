@@ -45,6 +45,9 @@ enum Finalize {
     FIN_STOP = 4,
     // S[S_DELTA_OLD] = S[S_DELTA]; S[S_DELTA] = sum, never counted
     FIN_DELTA_NOCOUNT = 5,
+    // MINRES, two sums in one finishing block: FIN_STOP of the update's
+    // (partials2, nb2), then FIN_DELTA_NOCOUNT of the operator's
+    FIN_STOP_DELTA = 6,
 };
 
 struct Reduce {
@@ -57,6 +60,9 @@ struct Reduce {
     // and sets S[S_DONE] when |r.z| <= S[S_THRESH].  The host can then queue
     // several iterations between synchronisations.
     int guard;
+    // FIN_STOP_DELTA: the partials an earlier launch left (one value each)
+    const double *partials2;
+    unsigned nb2;
 };
 
 // Scalar density field (EBE only): element e's local matrices are scaled by
@@ -134,6 +140,15 @@ struct Jac {
     const T *dinv;
     T vinv, pinv;
     const T *btab;
+    const uint8_t *bkeys;
+    uint32_t nvel;
+};
+
+// The Stokes Jacobi diagonal by DOF class (JAC_FLUID), for the MINRES vector
+// kernels in either precision: the values the stored diagonal holds.
+struct FluidJac {
+    double vinv, pinv;
+    const double *btab;
     const uint8_t *bkeys;
     uint32_t nvel;
 };
@@ -221,12 +236,17 @@ template <typename T> void launch_sub_precond(T *r, const T *q, const T *dinv, T
                                               hipStream_t s);
 // MINRES: dnew = rt + b dold (dnew may be dold) ; q = s + b q ; reduce q.(dinv q) ;
 // b = S[DELTA]/S[DELTA_OLD] (first: d = rt, q = s)
+// (J non-null: M^-1 by DOF class, dinv is not read)
 template <typename T> void launch_minres_dir(const T *dold, T *dnew, T *q, const T *rt, const T *sv, const T *dinv,
-                                             const double *S, int first, const Reduce *red, size_t n, hipStream_t s);
+                                             const FluidJac *J, const double *S, int first, const Reduce *red,
+                                             size_t n, hipStream_t s);
 // MINRES: rn = rt/dinv - a q ; rt = dinv rn ; x += a d (x == nullptr: the
 // iterate is left to the direction ring's flush) ; reduce rn.rt
-template <typename T> void launch_minres_update(T *x, T *rt, const T *d, const T *q, const T *dinv, const Reduce *red,
-                                                size_t n, hipStream_t s);
+// (finish false: the partials stay for a FIN_STOP_DELTA finish; returns their
+// number)
+template <typename T> unsigned launch_minres_update(T *x, T *rt, const T *d, const T *q, const T *dinv,
+                                                    const FluidJac *J, const Reduce *red, size_t n, hipStream_t s,
+                                                    bool finish = true);
 // FP64 outer refinement: x64 += e32
 void launch_add_correction(double *x, const float *e, size_t n, hipStream_t s);
 // y += x

@@ -425,13 +425,40 @@ __global__ void __launch_bounds__(BS) k_sub_precond(T *__restrict__ r, const T *
     store_partials<1>(red, vv);
 }
 
+// CLS: M^-1 by DOF class instead of a stored diagonal (Stokes: velocity, pore
+// pressure, border pressure by its node's fluid key): the same values, one
+// vector pass less in each of the two kernels (256^3 FP64: @DIR@ and @UPD@).
+template <typename T>
+__device__ __forceinline__ V16<T> ld_inv(const FluidJac &J, const T *__restrict__ dinv, size_t o, bool cls)
+{
+    constexpr int W = V16<T>::W;
+    if (!cls) return ld16(dinv + o);
+    V16<T> m;
+    const size_t nv3 = 3 * (size_t)J.nvel, nv4 = 4 * (size_t)J.nvel;
+#pragma unroll
+    for (int k = 0; k < W; k++) m.e[k] = o + k < nv3 ? (T)J.vinv : (T)J.pinv;
+    if (o + W > nv4) {
+#pragma unroll
+        for (int k = 0; k < W; k++)
+            if (o + k >= nv4) m.e[k] = (T)J.btab[J.bkeys[o + k - nv4]];
+    }
+    return m;
+}
+template <typename T>
+__device__ __forceinline__ T inv_at(const FluidJac &J, const T *__restrict__ dinv, size_t i, bool cls)
+{
+    if (!cls) return dinv[i];
+    const size_t nv3 = 3 * (size_t)J.nvel, nv4 = 4 * (size_t)J.nvel;
+    return i < nv3 ? (T)J.vinv : (i < nv4 ? (T)J.pinv : (T)J.btab[J.bkeys[i - nv4]]);
+}
+
 // MINRES: d = rt + b dold (written to dnew, which may be dold) ; q = s + b q ;
 // reduce q.(dinv q)
-template <typename T>
+template <typename T, bool CLS>
 __global__ void __launch_bounds__(BS) k_minres_dir(const T *dold, T *dnew, T *__restrict__ q,
                                                    const T *__restrict__ rt, const T *__restrict__ sv,
                                                    const T *__restrict__ dinv, const double *__restrict__ S, int first,
-                                                   size_t n, Reduce red)
+                                                   size_t n, Reduce red, FluidJac J)
 {
     if (stopped(red)) return;
     const T b = first ? T(0) : (T)(S[S_DELTA] / S[S_DELTA_OLD]);
@@ -440,7 +467,7 @@ __global__ void __launch_bounds__(BS) k_minres_dir(const T *dold, T *dnew, T *__
     FOR_VECTORS
     {
         const size_t o = j_ * W_;
-        const V16<T> rv = ld16(rt + o), s_ = ld16(sv + o), mv = ld16(dinv + o);
+        const V16<T> rv = ld16(rt + o), s_ = ld16(sv + o), mv = ld_inv<T>(J, dinv, o, CLS);
         V16<T> dv = ld16(dold + o), qv = ld16(q + o);
 #pragma unroll
         for (int k = 0; k < W_; k++) {
@@ -457,7 +484,7 @@ __global__ void __launch_bounds__(BS) k_minres_dir(const T *dold, T *dnew, T *__
         const T qn = first ? sv[i] : sv[i] + b * q[i];
         dnew[i] = dn;
         q[i] = qn;
-        acc += (double)qn * (double)(dinv[i] * qn);
+        acc += (double)qn * (double)(inv_at<T>(J, dinv, i, CLS) * qn);
     }
     double vv[1] = {acc};
     store_partials<1>(red, vv);
@@ -465,10 +492,10 @@ __global__ void __launch_bounds__(BS) k_minres_dir(const T *dold, T *dnew, T *__
 
 // MINRES: rn = rt/dinv - a q ; rt = dinv rn ; (XU) x += a d ; reduce rn.rt.
 // Without XU the iterate is left to the direction ring's flush.
-template <typename T, bool XU>
+template <typename T, bool XU, bool CLS>
 __global__ void __launch_bounds__(BS) k_minres_update(T *__restrict__ x, T *__restrict__ rt, const T *__restrict__ d,
                                                       const T *__restrict__ q, const T *__restrict__ dinv, size_t n,
-                                                      Reduce red)
+                                                      Reduce red, FluidJac J)
 {
     if (stopped(red)) return;
     const T a = (T)red.S[S_ALPHA];
@@ -478,7 +505,7 @@ __global__ void __launch_bounds__(BS) k_minres_update(T *__restrict__ x, T *__re
     {
         const size_t o = j_ * W_;
         V16<T> rv = ld16(rt + o);
-        const V16<T> qv = ld16(q + o), mv = ld16(dinv + o);
+        const V16<T> qv = ld16(q + o), mv = ld_inv<T>(J, dinv, o, CLS);
 #pragma unroll
         for (int k = 0; k < W_; k++) {
             const T rn = rv.e[k] / mv.e[k] - a * qv.e[k];
@@ -496,8 +523,9 @@ __global__ void __launch_bounds__(BS) k_minres_update(T *__restrict__ x, T *__re
     }
     FOR_TAIL(n)
     {
-        const T rn = rt[i] / dinv[i] - a * q[i];
-        const T rtn = dinv[i] * rn;
+        const T mi = inv_at<T>(J, dinv, i, CLS);
+        const T rn = rt[i] / mi - a * q[i];
+        const T rtn = mi * rn;
         rt[i] = rtn;
         if constexpr (XU) x[i] += a * d[i];
         acc += (double)rn * (double)rtn;
@@ -1148,7 +1176,7 @@ static inline int stream_grid(size_t n, size_t elem_bytes)
     return b < 1 ? 1 : (int)b;
 }
 
-static Reduce noreduce() { Reduce r; r.partials = nullptr; r.S = nullptr; r.fin = 0; r.slot = 0; r.guard = 0; return r; }
+static Reduce noreduce() { Reduce r; r.partials = nullptr; r.S = nullptr; r.fin = 0; r.slot = 0; r.guard = 0; r.partials2 = nullptr; r.nb2 = 0; return r; }
 
 // One block, bound by latency alone: the partials were written by all XCDs,
 // so every read misses this XCD's L2 (about 0.8 us).  The 16 wavefronts share
@@ -1162,13 +1190,12 @@ __global__ void __launch_bounds__(1024) k_reduce_finish(Reduce red, unsigned nb)
 {
     constexpr int WAVES = 16, PER = NV <= 1 ? 16 : (NV == 2 ? 8 : (NV <= 4 ? 4 : 2));  // wavefronts per value
     constexpr int TURN = 8;
-    __shared__ double part[WAVES];
+    __shared__ double part[WAVES], part2[WAVES];
     double *S = red.S;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, k = w / PER;
     const double done = red.guard ? S[S_DONE] : 0.0;
     const double delta_cur = S[S_DELTA], delta_old = S[S_DELTA_OLD], iter = S[S_ITER], thresh = S[S_THRESH];
-    if (k < NV) {
-        const double *p = red.partials + (size_t)k * nb;
+    auto list_sum = [&](const double *p, unsigned nb) -> double {
         double sum = 0;
         for (unsigned b0 = (w % PER) * 64 + lane; b0 < nb; b0 += PER * 64 * TURN) {
             double a[TURN];
@@ -1180,8 +1207,15 @@ __global__ void __launch_bounds__(1024) k_reduce_finish(Reduce red, unsigned nb)
 #pragma unroll
             for (int t = 0; t < TURN; t++) sum += a[t];
         }
-        sum = wave_sum(sum);
+        return wave_sum(sum);
+    };
+    if (k < NV) {
+        const double sum = list_sum(red.partials + (size_t)k * nb, nb);
         if (lane == 0) part[w] = sum;
+    }
+    if (NV == 1 && red.partials2) {
+        const double sum = list_sum(red.partials2, red.nb2);
+        if (lane == 0) part2[w] = sum;
     }
     __syncthreads();
     if (threadIdx.x != 0 || done != 0.0) return;
@@ -1230,6 +1264,17 @@ __global__ void __launch_bounds__(1024) k_reduce_finish(Reduce red, unsigned nb)
             if (fabs(s[0]) <= thresh) S[S_DONE] = 1.0;
         }
     } else if (red.fin == FIN_DELTA_NOCOUNT) {
+        S[S_DELTA_OLD] = delta_cur;
+        S[S_DELTA] = s[0];
+    } else if (red.fin == FIN_STOP_DELTA) {
+        double stop = 0;
+#pragma unroll
+        for (int i = 0; i < WAVES; i++) stop += part2[i];
+        S[S_STOP] = stop;
+        if (red.guard) {
+            S[S_ITER] = iter + 1.0;
+            if (fabs(stop) <= thresh) S[S_DONE] = 1.0;
+        }
         S[S_DELTA_OLD] = delta_cur;
         S[S_DELTA] = s[0];
     } else {
@@ -1385,19 +1430,27 @@ void launch_sub_precond(T *r, const T *q, const T *dinv, T *z, const Reduce *red
 }
 
 template <typename T>
-void launch_minres_dir(const T *dold, T *dnew, T *q, const T *rt, const T *sv, const T *dinv, const double *S,
-                       int first, const Reduce *red, size_t n, hipStream_t s)
+void launch_minres_dir(const T *dold, T *dnew, T *q, const T *rt, const T *sv, const T *dinv, const FluidJac *J,
+                       const double *S, int first, const Reduce *red, size_t n, hipStream_t s)
 {
-    LAUNCH_RED(1, k_minres_dir<T>, stream_grid(n, sizeof(T)), s, *red, dold, dnew, q, rt, sv, dinv, S, first, n,
-               *red);
+    const int grid = stream_grid(n, sizeof(T));
+    if (J) LAUNCH_RED(1, (k_minres_dir<T, true>), grid, s, *red, dold, dnew, q, rt, sv, dinv, S, first, n, *red, *J);
+    else LAUNCH_RED(1, (k_minres_dir<T, false>), grid, s, *red, dold, dnew, q, rt, sv, dinv, S, first, n, *red,
+                    FluidJac{});
 }
 
 template <typename T>
-void launch_minres_update(T *x, T *rt, const T *d, const T *q, const T *dinv, const Reduce *red, size_t n,
-                          hipStream_t s)
+unsigned launch_minres_update(T *x, T *rt, const T *d, const T *q, const T *dinv, const FluidJac *J, const Reduce *red,
+                              size_t n, hipStream_t s, bool finish)
 {
-    if (x) LAUNCH_RED(1, (k_minres_update<T, true>), stream_grid(n, sizeof(T)), s, *red, x, rt, d, q, dinv, n, *red);
-    else LAUNCH_RED(1, (k_minres_update<T, false>), stream_grid(n, sizeof(T)), s, *red, x, rt, d, q, dinv, n, *red);
+    const unsigned grid = (unsigned)stream_grid(n, sizeof(T));
+    const FluidJac none{};
+    if (x && J) k_minres_update<T, true, true><<<grid, BS, 0, s>>>(x, rt, d, q, dinv, n, *red, *J);
+    else if (x) k_minres_update<T, true, false><<<grid, BS, 0, s>>>(x, rt, d, q, dinv, n, *red, none);
+    else if (J) k_minres_update<T, false, true><<<grid, BS, 0, s>>>(x, rt, d, q, dinv, n, *red, *J);
+    else k_minres_update<T, false, false><<<grid, BS, 0, s>>>(x, rt, d, q, dinv, n, *red, none);
+    if (finish) launch_reduce_finish(*red, grid, 1, s);
+    return grid;
 }
 
 // Key-Jacobi launchers: one block per contiguous range of 4-node groups
@@ -1603,10 +1656,10 @@ void launch_interpl2(const double *coarse, double *fine, int rows, int cols, int
     template void launch_pcg_dir<T>(T *, const T *, const double *, int, size_t, hipStream_t, int);           \
     template void launch_pcg_update<T>(T *, T *, const T *, T *, const T *, const Reduce *, size_t, hipStream_t); \
     template void launch_sub_precond<T>(T *, const T *, const T *, T *, const Reduce *, size_t, hipStream_t); \
-    template void launch_minres_dir<T>(const T *, T *, T *, const T *, const T *, const T *, const double *, int, \
-                                       const Reduce *, size_t, hipStream_t);                                  \
-    template void launch_minres_update<T>(T *, T *, const T *, const T *, const T *, const Reduce *, size_t,  \
-                                          hipStream_t);                                                       \
+    template void launch_minres_dir<T>(const T *, T *, T *, const T *, const T *, const T *, const FluidJac *, \
+                                       const double *, int, const Reduce *, size_t, hipStream_t);             \
+    template unsigned launch_minres_update<T>(T *, T *, const T *, const T *, const T *, const FluidJac *,      \
+                                              const Reduce *, size_t, hipStream_t, bool);                     \
     template void launch_dot<T>(const T *, const T *, size_t, const Reduce *, hipStream_t);                   \
     template void launch_fluid_velocity_sum<T>(const OpDesc &, const T *, const Reduce *, hipStream_t);       \
     template void launch_kj_precond<T>(const OpDesc &, const T *, T *, const Reduce *, hipStream_t);          \

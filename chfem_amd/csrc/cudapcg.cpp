@@ -58,6 +58,12 @@ struct Solver {
     // w = 0: not set up yet), per precision
     double *ring64[RING_MAX] = {};
     float *ring32[RING_MAX] = {};
+    // device memory behind the ring slots, and behind the CG / MINRES vectors
+    // of a precision (d, q, s, z2, q2, dinv; FP32 with x, r): one allocation
+    // each, since freeing costs about 0.3 ms per allocation whatever its size
+    std::vector<void *> ring_blocks;
+    double *vec_block64 = nullptr;
+    float *vec_block32 = nullptr;
     int ring_w64 = 0, ring_w32 = 0;
     unsigned ring_try64 = 0, ring_try32 = 0;  // widest ring asked for so far
     bool arrays = false, user_arrays = false, x0_set = false, dinv_valid = false;
@@ -283,13 +289,22 @@ static cudapcgFlag_t free_solver_arrays()
 {
     if (!g) return CUDAPCG_FALSE;
     if (!g->x0_set) dfree(g->x64);
-    dfree(g->d64); dfree(g->q64); dfree(g->s64); dfree(g->dinv64);
-    dfree(g->x32); dfree(g->r32); dfree(g->d32); dfree(g->q32); dfree(g->s32); dfree(g->dinv32);
-    dfree(g->z2_64); dfree(g->q2_64); dfree(g->z2_32); dfree(g->q2_32);
+    if (g->vec_block64) {
+        dfree(g->vec_block64);
+        g->d64 = g->q64 = g->s64 = g->z2_64 = g->q2_64 = g->dinv64 = nullptr;
+    }
+    dfree(g->d64); dfree(g->q64); dfree(g->dinv64);  // the lean solvers'
+    dfree(g->vec_block32);
+    g->x32 = g->r32 = g->d32 = g->q32 = g->s32 = g->z2_32 = g->q2_32 = g->dinv32 = nullptr;
     dfree(g->dnode64); dfree(g->dnode32);
     dfree(g->xr64); dfree(g->hist);
     g->xr_n = g->hist_n = 0;
-    for (int k = 0; k < RING_MAX; k++) { dfree(g->ring64[k]); dfree(g->ring32[k]); }
+    for (void *b : g->ring_blocks) (void)hipFree(b);
+    g->ring_blocks.clear();
+    for (int k = 0; k < RING_MAX; k++) {
+        g->ring64[k] = nullptr;
+        g->ring32[k] = nullptr;
+    }
     g->ring_w64 = g->ring_w32 = 0;
     g->ring_try64 = g->ring_try32 = 0;
     dfree(g->partials); dfree(g->S);
@@ -301,13 +316,16 @@ static cudapcgFlag_t free_solver_arrays()
     return CUDAPCG_TRUE;
 }
 
+// entries between vectors of one allocation: whole 4 KiB pages
+template <typename T> static size_t vec_stride(size_t n) { return (n * sizeof(T) + 4095) / 4096 * 4096 / sizeof(T); }
+
 static bool is_lean();
 static bool is_two_vector();
 static cudapcgFlag_t alloc_solver_arrays()
 {
     if (!g || !g->model) return CUDAPCG_FALSE;
     const size_t n = nvars();
-    const size_t b8 = n * sizeof(double), b4 = n * sizeof(float);
+    const size_t b8 = n * sizeof(double);
     if (is_lean()) {
         // memory-lean solvers: z (the RHS buffer) and d, plus x for CG3 and
         // MINRES3; a stored diagonal or an operator work vector only where
@@ -316,22 +334,25 @@ static cudapcgFlag_t alloc_solver_arrays()
         if (!g->d64) CHECK_HIP(hipMalloc(&g->d64, b8));
     } else {
     if (!g->x64) CHECK_HIP(hipMalloc(&g->x64, b8));
-    if (!g->d64) CHECK_HIP(hipMalloc(&g->d64, b8));
-    if (!g->q64) CHECK_HIP(hipMalloc(&g->q64, b8));
-    // s: MINRES's A M^-1 r, or CG's second direction buffer (fused direction update)
-    if (!g->s64) CHECK_HIP(hipMalloc(&g->s64, b8));
-    if (!g->z2_64) CHECK_HIP(hipMalloc(&g->z2_64, b8));
-    if (!g->q2_64) CHECK_HIP(hipMalloc(&g->q2_64, b8));
-    if (!g->dinv64) CHECK_HIP(hipMalloc(&g->dinv64, b8));
-    if (g->precision == CHFEM_PREC_MIXED) {
-        if (!g->x32) CHECK_HIP(hipMalloc(&g->x32, b4));
-        if (!g->r32) CHECK_HIP(hipMalloc(&g->r32, b4));
-        if (!g->d32) CHECK_HIP(hipMalloc(&g->d32, b4));
-        if (!g->q32) CHECK_HIP(hipMalloc(&g->q32, b4));
-        if (!g->s32) CHECK_HIP(hipMalloc(&g->s32, b4));
-        if (!g->z2_32) CHECK_HIP(hipMalloc(&g->z2_32, b4));
-        if (!g->q2_32) CHECK_HIP(hipMalloc(&g->q2_32, b4));
-        if (!g->dinv32) CHECK_HIP(hipMalloc(&g->dinv32, b4));
+    if (!g->vec_block64) {
+        const size_t st = vec_stride<double>(n);
+        CHECK_HIP(hipMalloc(&g->vec_block64, 6 * st * sizeof(double)));
+        double *p = g->vec_block64;
+        // s: MINRES's A M^-1 r, or CG's second direction buffer (fused
+        // direction update)
+        for (double **v : {&g->d64, &g->q64, &g->s64, &g->z2_64, &g->q2_64, &g->dinv64}) {
+            *v = p;
+            p += st;
+        }
+    }
+    if (g->precision == CHFEM_PREC_MIXED && !g->vec_block32) {
+        const size_t st = vec_stride<float>(n);
+        CHECK_HIP(hipMalloc(&g->vec_block32, 8 * st * sizeof(float)));
+        float *p = g->vec_block32;
+        for (float **v : {&g->x32, &g->r32, &g->d32, &g->q32, &g->s32, &g->z2_32, &g->q2_32, &g->dinv32}) {
+            *v = p;
+            p += st;
+        }
     }
     }
     const size_t pn = (size_t)MAX_PARTIAL_BLOCKS * 8;
@@ -638,12 +659,18 @@ static Ring<T> dir_ring(T *d, T *s, unsigned cap)
         if (!getenv("CHFEM_RING") && vb && hipMemGetInfo(&freeb, &totb) == hipSuccess)
             want = (unsigned)std::min<size_t>(want, std::max(w, 2) + freeb / 4 / vb);
         if (w < 2) w = 2;
-        for (unsigned k = (unsigned)w; k < want; k++) {
-            if (hipMalloc(&extra[k], vb) != hipSuccess) {
+        // one allocation for the slots still wanted, or for half as many
+        const size_t st = vec_stride<T>(nvars());
+        for (unsigned more = want > (unsigned)w ? want - (unsigned)w : 0u; more > 0; more /= 2) {
+            void *b = nullptr;
+            if (hipMalloc(&b, more * st * sizeof(T)) != hipSuccess) {
                 (void)hipGetLastError();
-                break;
+                continue;
             }
-            w = (int)k + 1;
+            g->ring_blocks.push_back(b);
+            for (unsigned k = 0; k < more; k++) extra[w + k] = (T *)b + k * st;
+            w += (int)more;
+            break;
         }
     }
     Ring<T> r{};

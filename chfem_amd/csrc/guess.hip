@@ -176,19 +176,111 @@ void conv(int mode, const uint16_t *in, Grid3 gi, int Ci, const uint16_t *W, con
 }
 
 // ---------------------------------------------------------------------------
-// weight gradients: block (chunk of output voxels, tap); the Co x Ci tile of
-// the tap is split into 16x16 products spread over the 4 wavefronts
+// weight gradients
 // ---------------------------------------------------------------------------
-// output voxels per block: 2048, halved (down to 256) while the launch
-// would have fewer than 2048 blocks, so the coarse levels' few voxels are
-// still spread over the GPU
+// output voxels per block.  3x3x3 layers: about 256 chunks, in multiples of
+// the 64 voxels that a block's wavefronts take per step.  DOWN: 2048, halved
+// (down to 256) while the launch would have fewer than 2048 blocks, so the
+// coarse levels' few voxels are still spread over the GPU.
 static int wchunk(size_t V, int taps)
 {
+    if (taps == 27) {
+        const size_t c = ((V + 255) / 256 + 63) / 64 * 64;
+        return (int)(c < 64 ? 64 : c);
+    }
     int c = 2048;
     while (c > 256 && ((V + c - 1) / c) * (size_t)taps < 2048) c /= 2;
     return c;
 }
 
+// 3x3x3 layers (SAME, UP).  A block takes a chunk of output voxels, one layer
+// offset dl of the taps (blockIdx.y) and 16 input channels (blockIdx.z); a
+// wavefront keeps the products of its 9 taps and all NCO * 16 output channels
+// in registers, so a voxel's output gradients are read once for 9 taps, and
+// per column offset the 6 rows around 4 consecutive voxels once for the 3 row
+// offsets (for row counts that are multiples of 4: 4 consecutive voxels share
+// a column).  The wavefronts take every fourth 16 voxels and add up through
+// LDS.  Bound by its 2-byte gathers: 54 input loads per 27 products, where a
+// block per tap read 27 x 8 and formed every voxel's position for every tap.
+// 64^3, 16 -> 16: 39 us, up-convolution 32 -> 16: 56 us (403, 463 before).
+template <int MODE, int NCO>
+__global__ void __launch_bounds__(NB) k_convw27(const uint16_t *__restrict__ in, Grid3 gi, int Ci,
+                                                const uint16_t *__restrict__ dz, Grid3 go, int chunk,
+                                                float *__restrict__ part)
+{
+    constexpr int Co = NCO * 16;
+    __shared__ float4_t red[3][9][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i = lane & 15, kg = lane >> 4;
+    const int dl = (int)blockIdx.y - 1, cit = blockIdx.z;
+    const uint32_t V = (uint32_t)go.ny * go.nx * go.nz;
+    const uint32_t v0 = blockIdx.x * (uint32_t)chunk, v1 = v0 + chunk < V ? v0 + chunk : V;
+    float4_t acc[9][NCO];
+#pragma unroll
+    for (int t = 0; t < 9; t++)
+#pragma unroll
+        for (int m = 0; m < NCO; m++) acc[t][m] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (uint32_t vk = v0 + 16 * (uint32_t)wave; vk < v1; vk += 64) {
+        // this lane's 4 voxels (all in the chunk or all past it)
+        const uint32_t vq = vk + 4 * kg;
+        const bool ok = vq < v1;
+        const uint32_t v = ok ? vq : v0;
+        const uint32_t cl = v / (uint32_t)go.ny;
+        const int r = (int)(v - cl * (uint32_t)go.ny), l = (int)(cl / (uint32_t)go.nx), c = (int)(cl - (uint32_t)l * go.nx);
+        short4_t az[NCO];
+#pragma unroll
+        for (int m = 0; m < NCO; m++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const short g = (short)dz[(size_t)(v + e) * Co + m * 16 + i];
+                az[m][e] = ok ? g : (short)0;
+            }
+        const int ll = wrap(l + dl, go.nz);
+        uint32_t row[6];
+#pragma unroll
+        for (int e = 0; e < 6; e++) {
+            const int rr = wrap(r + e - 1, go.ny);
+            row[e] = (uint32_t)(MODE == CONV_UP ? rr >> 1 : rr);
+        }
+#pragma unroll
+        for (int dc = 0; dc < 3; dc++) {
+            const int cc = wrap(c + dc - 1, go.nx);
+            const uint32_t col = MODE == CONV_UP ? ((uint32_t)(ll >> 1) * gi.nx + (uint32_t)(cc >> 1)) * gi.ny
+                                                 : ((uint32_t)ll * gi.nx + (uint32_t)cc) * gi.ny;
+            short x[6];
+#pragma unroll
+            for (int e = 0; e < 6; e++) x[e] = (short)in[(size_t)(col + row[e]) * Ci + cit * 16 + i];
+#pragma unroll
+            for (int dr = 0; dr < 3; dr++) {
+                const short4_t bx = {x[dr], x[dr + 1], x[dr + 2], x[dr + 3]};
+#pragma unroll
+                for (int m = 0; m < NCO; m++) acc[3 * dc + dr][m] = mfma16(az[m], bx, acc[3 * dc + dr][m]);
+            }
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < NCO; m++) {
+        if (wave > 0)
+#pragma unroll
+            for (int t = 0; t < 9; t++) red[wave - 1][t][lane] = acc[t][m];
+        __syncthreads();
+        if (wave == 0)
+#pragma unroll
+            for (int t = 0; t < 9; t++) {
+                const float4_t sum = (acc[t][m] + red[0][t][lane]) + (red[1][t][lane] + red[2][t][lane]);
+                const int tap = 9 * (int)blockIdx.y + t;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int co = m * 16 + 4 * kg + e, ci = cit * 16 + i;
+                    part[(((size_t)blockIdx.x * 27 + tap) * Co + co) * Ci + ci] = sum[e];
+                }
+            }
+        __syncthreads();
+    }
+}
+
+// DOWN layers, and 3x3x3 ones on grids whose row count is no multiple of 4:
+// block (chunk of output voxels, tap); the Co x Ci tile of the tap is split into 16x16 products spread over the 4 wavefronts
 template <int MODE>
 __global__ void __launch_bounds__(NB) k_convw(const uint16_t *__restrict__ in, Grid3 gi, int Ci,
                                               const uint16_t *__restrict__ dz, Grid3 go, int Co, int taps,
@@ -262,24 +354,47 @@ __global__ void __launch_bounds__(NB) k_convw(const uint16_t *__restrict__ in, G
     }
 }
 
+// Adds the chunks' partials: 32 outputs per block, the chunks shared by its 8
+// groups of 32 work-items, 8 reads of each in flight (one work-item per
+// output reading chunk after chunk took 42 us on 128 chunks of 6912; now
+// 4.6 on 256).
 __global__ void __launch_bounds__(NB) k_wsum(const float *__restrict__ part, int nchunk, int taps, int Co, int Ci,
                                              float *__restrict__ grad)
 {
+    constexpr int OUTS = 32, GROUPS = NB / OUTS, TURN = 8;
+    __shared__ float red[GROUPS][OUTS];
     const size_t n = (size_t)taps * Co * Ci;
-    for (size_t j = (size_t)blockIdx.x * NB + threadIdx.x; j < n; j += (size_t)gridDim.x * NB) {
-        // j enumerates (co, t, ci) in the master layout
-        const int ci = (int)(j % Ci), t = (int)((j / Ci) % taps), co = (int)(j / ((size_t)Ci * taps));
-        float sum = 0.f;
-        for (int ch = 0; ch < nchunk; ch++) sum += part[(((size_t)ch * taps + t) * Co + co) * Ci + ci];
-        grad[j] += sum;
-    }
+    const int o = threadIdx.x % OUTS, g = threadIdx.x / OUTS;
+    // p enumerates the partials' layout (t, co, ci)
+    const size_t p = (size_t)blockIdx.x * OUTS + o;
+    float sum = 0.f;
+    if (p < n)
+        for (int c0 = g; c0 < nchunk; c0 += GROUPS * TURN) {
+            float a[TURN];
+#pragma unroll
+            for (int k = 0; k < TURN; k++) {
+                const int ch = c0 + k * GROUPS;
+                a[k] = ch < nchunk ? part[(size_t)ch * n + p] : 0.f;
+            }
+#pragma unroll
+            for (int k = 0; k < TURN; k++) sum += a[k];
+        }
+    red[g][o] = sum;
+    __syncthreads();
+    if (g != 0 || p >= n) return;
+#pragma unroll
+    for (int k = 1; k < GROUPS; k++) sum += red[k][o];
+    const int ci = (int)(p % Ci), co = (int)((p / Ci) % Co), t = (int)(p / ((size_t)Ci * Co));
+    grad[((size_t)co * taps + t) * Ci + ci] += sum;
 }
 
+// (an upper bound that grows with the grid: the scratch of a grid also serves
+// every smaller one)
 size_t wpart_size(Grid3 go, int Co, int Ci, int taps)
 {
     const size_t V = (size_t)go.ny * go.nx * go.nz;
-    const int c = wchunk(V, taps);
-    return ((V + c - 1) / c) * (size_t)taps * Co * Ci;
+    const size_t most = taps == 27 ? 256 : V / 2048 + 512, all = (V + 63) / 64;
+    return (most < all ? most : all) * taps * Co * Ci;
 }
 
 void conv_wgrad(int mode, const uint16_t *in, Grid3 gi, int Ci, const uint16_t *dz, Grid3 go, int Co, float *part,
@@ -289,12 +404,24 @@ void conv_wgrad(int mode, const uint16_t *in, Grid3 gi, int Ci, const uint16_t *
     const size_t V = (size_t)go.ny * go.nx * go.nz;
     const int chunk = wchunk(V, taps);
     const int nchunk = (int)((V + chunk - 1) / chunk);
-    dim3 grid(nchunk, taps);
-    if (mode == CONV_SAME) k_convw<CONV_SAME><<<grid, NB, 0, s>>>(in, gi, Ci, dz, go, Co, taps, chunk, part);
-    else if (mode == CONV_DOWN) k_convw<CONV_DOWN><<<grid, NB, 0, s>>>(in, gi, Ci, dz, go, Co, taps, chunk, part);
-    else k_convw<CONV_UP><<<grid, NB, 0, s>>>(in, gi, Ci, dz, go, Co, taps, chunk, part);
+    if (mode == CONV_DOWN) {
+        k_convw<CONV_DOWN><<<dim3(nchunk, taps), NB, 0, s>>>(in, gi, Ci, dz, go, Co, taps, chunk, part);
+    } else if (go.ny % 4) {
+        // (4 consecutive voxels straddle columns: the coarse levels of row
+        // counts like 24 or 40)
+        if (mode == CONV_SAME) k_convw<CONV_SAME><<<dim3(nchunk, taps), NB, 0, s>>>(in, gi, Ci, dz, go, Co, taps, chunk, part);
+        else k_convw<CONV_UP><<<dim3(nchunk, taps), NB, 0, s>>>(in, gi, Ci, dz, go, Co, taps, chunk, part);
+    } else {
+        const dim3 grid(nchunk, 3, Ci / 16);
+#define CONVW_CASE(M, N) \
+    if (mode == M && Co == N * 16) k_convw27<M, N><<<grid, NB, 0, s>>>(in, gi, Ci, dz, go, chunk, part);
+        CONVW_CASE(CONV_SAME, 1) CONVW_CASE(CONV_SAME, 2) CONVW_CASE(CONV_SAME, 3)
+        CONVW_CASE(CONV_UP, 1) CONVW_CASE(CONV_UP, 2) CONVW_CASE(CONV_UP, 3)
+#undef CONVW_CASE
+        if (Co > 48) fprintf(stderr, "chfem guess: no weight-gradient kernel for %d output channels\n", Co);
+    }
     const size_t n = (size_t)taps * Co * Ci;
-    k_wsum<<<(unsigned)((n + NB - 1) / NB), NB, 0, s>>>(part, nchunk, taps, Co, Ci, grad);
+    k_wsum<<<(unsigned)((n + 31) / 32), NB, 0, s>>>(part, nchunk, taps, Co, Ci, grad);
 }
 
 // ---------------------------------------------------------------------------
@@ -320,17 +447,17 @@ void pack_weights(const float *Wm, uint16_t *out, int Co, int Ci, int taps, int 
 }
 
 // ---------------------------------------------------------------------------
-// voxels per block of the activation backward (enough blocks at 64^3 and
-// below, where training runs)
-#define ACHUNK 256
+// voxels per block of the activation backward: 256, on the coarse levels 32
+// (16^3, 48 channels: 16 blocks of 51 serial steps took 25 us)
+static int achunk(size_t V) { return V >= 65536 ? 256 : 32; }
 
 __global__ void __launch_bounds__(NB) k_act_bwd(const float *__restrict__ dy, const uint16_t *__restrict__ y, int relu,
                                                 uint16_t *__restrict__ dz, float *__restrict__ skip_grad,
-                                                float *__restrict__ bpart, size_t V, int C)
+                                                float *__restrict__ bpart, size_t V, int C, int chunk)
 {
     __shared__ float red[NB];
     const int c = threadIdx.x % C, lanes = NB / C, vl = threadIdx.x / C;
-    const size_t v0 = (size_t)blockIdx.x * ACHUNK, v1 = v0 + ACHUNK < V ? v0 + ACHUNK : V;
+    const size_t v0 = (size_t)blockIdx.x * chunk, v1 = v0 + chunk < V ? v0 + chunk : V;
     float bsum = 0.f;
     if (vl < lanes) {
         for (size_t v = v0 + vl; v < v1; v += lanes) {
@@ -352,23 +479,32 @@ __global__ void __launch_bounds__(NB) k_act_bwd(const float *__restrict__ dy, co
     }
 }
 
-__global__ void k_bsum(const float *__restrict__ bpart, int nb, int C, float *__restrict__ bias_grad)
+// one block per channel (one work-item per channel adding block after block
+// took 65 us on 1024 blocks; now 4.6)
+__global__ void __launch_bounds__(NB) k_bsum(const float *__restrict__ bpart, int nb, int C,
+                                             float *__restrict__ bias_grad)
 {
-    const int c = threadIdx.x;
-    if (c >= C) return;
+    __shared__ float red[NB / 64];
+    const int c = blockIdx.x;
     float s = 0.f;
-    for (int b = 0; b < nb; b++) s += bpart[(size_t)b * C + c];
-    bias_grad[c] += s;
+#pragma unroll 4
+    for (int b = threadIdx.x; b < nb; b += NB) s += bpart[(size_t)b * C + c];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) bias_grad[c] += (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-size_t bias_part_size(size_t V, int C) { return ((V + ACHUNK - 1) / ACHUNK) * (size_t)C; }
+// (an upper bound that grows with V, as wpart_size)
+size_t bias_part_size(size_t V, int C) { return ((V < 65536 ? V : 65536) / 32 + V / 256 + 2) * (size_t)C; }
 
 void act_backward(const float *dy, const uint16_t *y, int relu, uint16_t *dz, float *skip_grad, float *bias_part,
                   float *bias_grad, size_t V, int C, hipStream_t s)
 {
-    const int nb = (int)((V + ACHUNK - 1) / ACHUNK);
-    k_act_bwd<<<nb, NB, 0, s>>>(dy, y, relu, dz, skip_grad, bias_part, V, C);
-    k_bsum<<<1, 64, 0, s>>>(bias_part, nb, C, bias_grad);
+    const int chunk = achunk(V), nb = (int)((V + chunk - 1) / chunk);
+    k_act_bwd<<<nb, NB, 0, s>>>(dy, y, relu, dz, skip_grad, bias_part, V, C, chunk);
+    k_bsum<<<C, NB, 0, s>>>(bias_part, nb, C, bias_grad);
 }
 
 // ---------------------------------------------------------------------------
@@ -401,7 +537,7 @@ void pool_children(const float *fine, Grid3 gf, float *coarse, int C, int accumu
 }
 
 // ---------------------------------------------------------------------------
-#define LCHUNK 512
+#define LCHUNK 128
 
 __global__ void __launch_bounds__(NB) k_mse(const float *__restrict__ y, int Cp, const float *__restrict__ target, int nt,
                                             size_t V, double scale, float *__restrict__ dy, double *__restrict__ part)
@@ -429,12 +565,14 @@ __global__ void __launch_bounds__(NB) k_mse(const float *__restrict__ y, int Cp,
     if (threadIdx.x == 0) part[blockIdx.x] = red[0] * scale;
 }
 
-__global__ void k_dsum(const double *__restrict__ part, int nb, double *__restrict__ out)
+__global__ void __launch_bounds__(64) k_dsum(const double *__restrict__ part, int nb, double *__restrict__ out)
 {
-    if (threadIdx.x != 0) return;
     double s = 0;
-    for (int b = 0; b < nb; b++) s += part[b];
-    *out += s;
+#pragma unroll 8
+    for (int b = threadIdx.x; b < nb; b += 64) s += part[b];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (threadIdx.x == 0) *out += s;
 }
 
 size_t loss_part_size(size_t V) { return (V + LCHUNK - 1) / LCHUNK; }

@@ -150,6 +150,65 @@ __global__ void __launch_bounds__(NB) k_conv(const uint16_t *__restrict__ in, Gr
         }
 }
 
+// Small grids: a wavefront takes 16 output voxels and 16 output channels, and
+// issues the loads of STEPS (tap, 16 input channels) steps before their
+// products, which keep k_conv's order (the same bits).  A 16^3 layer of 48
+// channels gave k_conv 64 wavefronts of 81 dependent steps each, bound by one
+// load latency per step: 115 us; here 23 us (8^3: 120 -> 23, 32^3
+// up-convolution 48 -> 32: 98 -> 47).  With enough voxels k_conv's 4 groups
+// per weight operand win.
+template <int MODE, bool OUTF>
+__global__ void __launch_bounds__(NB) k_conv_small(const uint16_t *__restrict__ in, Grid3 gi, int Ci,
+                                                   const uint16_t *__restrict__ W, int taps,
+                                                   const float *__restrict__ bias, const uint16_t *__restrict__ skip,
+                                                   int relu, void *out, int accumulate, Grid3 go, int Co)
+{
+    constexpr int STEPS = 9;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i = lane & 15, kg = lane >> 4;
+    const uint32_t V = (uint32_t)go.ny * go.nx * go.nz, NT = (uint32_t)Co / 16u;
+    const uint32_t job = blockIdx.x * 4u + wave, vb = job / NT * 16u, nt = job % NT;
+    if (vb >= V) return;  // no barriers in this kernel
+    const bool okA = vb + i < V;
+    const uint32_t va = okA ? vb + i : V - 1;
+    const int r = (int)(va % (uint32_t)go.ny), c = (int)(va / (uint32_t)go.ny % (uint32_t)go.nx),
+              l = (int)(va / ((uint32_t)go.ny * go.nx));
+    const int kc = Ci / 16, steps = taps * kc;
+    const uint16_t *wrow = W + (size_t)(nt * 16 + i) * ((size_t)taps * Ci) + 4 * kg;
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < steps; s0 += STEPS) {
+        short4_t a[STEPS], b[STEPS];
+#pragma unroll
+        for (int k = 0; k < STEPS; k++) {
+            // (steps past the last re-read it; their products are left out)
+            const int st = min(s0 + k, steps - 1), t = st / kc, c0 = (st - t * kc) * 16;
+            a[k] = *(const short4_t *)(in + in_index<MODE>(r, c, l, t, gi, go) * Ci + c0 + 4 * kg);
+            b[k] = *(const short4_t *)(wrow + (size_t)t * Ci + c0);
+            if (!okA) a[k] = short4_t{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int k = 0; k < STEPS; k++)
+            if (s0 + k < steps) acc = mfma16(a[k], b[k], acc);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const uint32_t vo = vb + 4 * kg + e;
+        if (vo >= V) continue;
+        const int co = nt * 16 + i;
+        float val = acc[e];
+        if (bias) val += bias[co];
+        if (skip) val += bf2f(skip[(size_t)vo * Co + co]);
+        if (relu) val = fmaxf(val, 0.f);
+        if (OUTF) {
+            float *o = (float *)out + (size_t)vo * Co + co;
+            *o = accumulate ? *o + val : val;
+        } else {
+            ((uint16_t *)out)[(size_t)vo * Co + co] = f2bf(val);
+        }
+    }
+}
+constexpr size_t CONV_SMALL = 65536;  // output voxels: 32^3 is faster here, 64^3 in k_conv
+
 void conv(int mode, const uint16_t *in, Grid3 gi, int Ci, const uint16_t *W, const float *bias, const uint16_t *skip,
           int relu, void *out, int out_f32, int accumulate, Grid3 go, int Co, hipStream_t s)
 {
@@ -157,6 +216,21 @@ void conv(int mode, const uint16_t *in, Grid3 gi, int Ci, const uint16_t *W, con
     const Grid3 rg = mode == CONV_PARITY ? gi : go;
     const size_t V = (size_t)rg.ny * rg.nx * rg.nz;
     dim3 grid((unsigned)((V + 64 * CG - 1) / (64 * CG)), mode == CONV_PARITY ? 8 : 1);
+    if (mode != CONV_PARITY && V <= CONV_SMALL && Co % 16 == 0) {
+        const unsigned sgrid = (unsigned)(((V + 15) / 16 * (Co / 16) + 3) / 4);
+#define CONV_SMALL_CASE(M)                                                                             \
+    if (mode == M) {                                                                                   \
+        if (out_f32)                                                                                   \
+            k_conv_small<M, true><<<sgrid, NB, 0, s>>>(in, gi, Ci, W, taps, bias, skip, relu, out, accumulate, go, Co); \
+        else                                                                                           \
+            k_conv_small<M, false><<<sgrid, NB, 0, s>>>(in, gi, Ci, W, taps, bias, skip, relu, out, accumulate, go, Co); \
+        return;                                                                                        \
+    }
+        CONV_SMALL_CASE(CONV_SAME)
+        CONV_SMALL_CASE(CONV_DOWN)
+        CONV_SMALL_CASE(CONV_UP)
+#undef CONV_SMALL_CASE
+    }
 #define CONV_CASE(M, NTv)                                                                              \
     if (mode == M && Co == NTv * 16) {                                                                 \
         if (out_f32)                                                                                   \

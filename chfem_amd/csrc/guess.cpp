@@ -56,9 +56,10 @@ struct Net {
     uint16_t *dz = nullptr;
     double *lpart = nullptr, *loss = nullptr;
     float *target = nullptr;
+    float *ypacked = nullptr;  // a prediction's outputs, packed for the host
     uint16_t *elem = nullptr;
     float *table = nullptr;
-    size_t cap_voxels = 0, cap_train = 0, cap_target = 0;
+    size_t cap_voxels = 0, cap_train = 0, cap_target = 0, cap_packed = 0;
     bool packed = false;
 };
 
@@ -351,6 +352,7 @@ void chfemGuessDestroy(void *h)
         dfree(n->act[a]);
         dfree(n->gact[a]);
     }
+    dfree(n->ypacked);
     dfree(n->y); dfree(n->gy); dfree(n->tmp); dfree(n->wpart); dfree(n->bpart); dfree(n->dz); dfree(n->lpart);
     dfree(n->loss); dfree(n->target); dfree(n->elem); dfree(n->table);
     dfree(n->w); dfree(n->g); dfree(n->m); dfree(n->v);
@@ -401,10 +403,16 @@ int chfemGuessPredict(void *h, const uint16_t *elem, const double *props, unsign
     const float *y = chfem::guess_predict_device(h, elem, props, nmat, nx, ny, nz, &C);
     if (!y) return 0;
     const size_t V = (size_t)nx * ny * nz;
-    std::vector<float> full(V * C);
-    if (!ok(hipMemcpyAsync(full.data(), y, full.size() * sizeof(float), hipMemcpyDeviceToHost, n->s))) return 0;
+    const size_t nt = V * n->nout;
+    if (nt > n->cap_packed) {
+        dfree(n->ypacked);
+        n->cap_packed = 0;
+        if (!ok(hipMalloc(&n->ypacked, nt * sizeof(float)))) return 0;
+        n->cap_packed = nt;
+    }
+    outputs(y, C, n->nout, V, n->ypacked, n->s);
+    if (!ok(hipMemcpyAsync(out, n->ypacked, nt * sizeof(float), hipMemcpyDeviceToHost, n->s))) return 0;
     if (!ok(hipStreamSynchronize(n->s))) return 0;
-    for (size_t v = 0; v < V; v++) memcpy(out + v * n->nout, full.data() + v * C, n->nout * sizeof(float));
     return 1;
 }
 

@@ -60,6 +60,9 @@ void adam(float *w, const float *g, float *m, float *v, size_t n, float lr, floa
 // input features: in[v][0..nf) = table[elem[v] * nf + k], other channels 0
 void features(const uint16_t *elem, const float *table, int nf, uint16_t *in, int C, size_t V, hipStream_t s);
 
+// the first n of every voxel's C outputs, packed
+void outputs(const float *y, int C, int n, size_t V, float *out, hipStream_t s);
+
 // x0[nd*i + a] = ramp of load case `load` at node i, component a, plus
 // scale * y[i][load*nd + a]
 void guess_to_x0(const float *y, int Cp, int load, int nd, Grid3 g, float scale, double *x0, hipStream_t s);

@@ -702,6 +702,26 @@ void features(const uint16_t *elem, const float *table, int nf, uint16_t *in, in
     k_features<<<b, NB, 0, s>>>(elem, table, nf, in, C, V);
 }
 
+// out[v * n + k] = y[v * C + k], k < n: the network's real outputs, packed for
+// the copy to the host (the padded channels are 14 of 32, and repacking on
+// the host cost as much again as the copy)
+__global__ void __launch_bounds__(NB) k_outputs(const float *__restrict__ y, int C, int n, size_t V,
+                                                float *__restrict__ out)
+{
+    const size_t all = V * n;
+    for (size_t j = (size_t)blockIdx.x * NB + threadIdx.x; j < all; j += (size_t)gridDim.x * NB) {
+        const size_t v = j / n;
+        out[j] = y[v * C + (j - v * n)];
+    }
+}
+
+void outputs(const float *y, int C, int n, size_t V, float *out, hipStream_t s)
+{
+    size_t b = (V * n + NB - 1) / NB;
+    if (b > 65536) b = 65536;
+    k_outputs<<<(unsigned)b, NB, 0, s>>>(y, C, n, V, out);
+}
+
 // load cases (seam axis, jumping component): X, Y, Z, YZ, XZ, XY
 __constant__ int cLoadAxis[6] = {0, 1, 2, 1, 2, 1};
 __constant__ int cLoadComp[6] = {0, 1, 2, 2, 0, 0};

@@ -4,19 +4,22 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <array>
+#include <vector>
+
 namespace chfem {
 namespace batch {
 
-// Walsh tile of the batched operators: 64 x 7 work-items own 64 node rows
-// (the halo-wavefront variant of walsh_tile: one more wavefront evaluates
-// the row above the tile), so 256 rows take 4 tiles; 512 work-items per block
-#define TILE_R 64
-#define TILE_C 7
-#define TILE_HALO true
-#define TILE_ROWS (TILE_HALO ? TILE_R : TILE_R - 1)
-#define TILE_THREADS (TILE_R * TILE_C + (TILE_HALO ? 64 : 0))
-// node layers per block
-#define TILE_LZ 32
+// Walsh tiles of the batched operators (walsh_tile): 64 x 7 with the halo
+// wavefront (64 owned rows), 32 x 8 (31 rows) and 64 x 8 (63 rows); one shape
+// and one number of node layers per block serve the whole batch
+// (batch_tile_rule)
+struct Shape {
+    int rows, cols;  // nodes owned per tile
+    int tr, tc;      // walsh_tile's TR (65: the halo variant) and TC
+};
+constexpr Shape SHAPES[] = {{64, 6, 65, 7}, {31, 7, 32, 8}, {63, 7, 64, 8}};
+constexpr int NSHAPES = 3;
 
 // one linear system (a load case of a sample), device view
 struct Sys {
@@ -61,6 +64,7 @@ enum { FIN_B_ALPHA = 0, FIN_B_DELTA, FIN_B_TRUE, FIN_B_DELTA0, FIN_B_START, FIN_
 
 struct Batch {
     int nsys = 0, nd = 1;
+    int shape = 0;             // of SHAPES
     const Sys *sys = nullptr;
     const Tile *tiles = nullptr;
     int ntiles = 0;
@@ -110,4 +114,9 @@ void apply_cg1(const Batch &b, float *z, float *z2, float *q, float *q2, float *
                hipStream_t s);
 
 }  // namespace batch
+
+// tile shape (index) and node layers per block for a batch of samples {ny,
+// nx, nz} with `loads` systems each, from the fitted tile cost (walsh.hip)
+int batch_tile_rule(bool elastic, const batch::Shape *shapes, int nshapes, const std::vector<std::array<int, 3>> &dims,
+                    int loads, int &lz);
 }  // namespace chfem

@@ -46,8 +46,8 @@ __device__ __forceinline__ bool selected(const double *Sb, int sys, int mode)
 // system's tiles (rows of tiles fastest): neighbouring tiles share an XCD's
 // L2, and every XCD keeps work while any system is still iterating.  Block
 // partials go to the tile's slot in its system's contiguous range.
-template <typename T, int ND, int TR, int TC>
-__global__ void __launch_bounds__(TR *TC + (TILE_HALO ? 64 : 0)) k_apply_walsh(const Sys *__restrict__ sys, const Tile *__restrict__ tiles,
+template <typename T, int ND, int TR, int TC, bool HALO>
+__global__ void __launch_bounds__(TR *TC + (HALO ? 64 : 0)) k_apply_walsh(const Sys *__restrict__ sys, const Tile *__restrict__ tiles,
                                                          const T *v, T *q, const double *__restrict__ Sb,
                                                          double *__restrict__ part, int mode)
 {
@@ -57,7 +57,7 @@ __global__ void __launch_bounds__(TR *TC + (TILE_HALO ? 64 : 0)) k_apply_walsh(c
     if (!selected<T>(Sb, t.sys, mode)) return;
     const Sys &S = sys[t.sys];
     const T *lamu = (const T *)(sizeof(T) == 4 ? S.mat32 : S.mat64);
-    const double d = walsh_tile<T, ND, TR, TC, true, 0, TILE_HALO>(v + S.off, q + S.off, S.keys, lamu, 0, S.ny, S.nx, S.nz, S.LZ,
+    const double d = walsh_tile<T, ND, TR, TC, true, 0, HALO>(v + S.off, q + S.off, S.keys, lamu, 0, S.ny, S.nx, S.nz, S.LZ,
                                                      t.bx, t.by, t.bz).dq;
     const double s = bsum(d);
     if (threadIdx.x == 0) part[t.slot] = s;
@@ -68,8 +68,8 @@ __global__ void __launch_bounds__(TR *TC + (TILE_HALO ? 64 : 0)) k_apply_walsh(c
 // each tile.  A system's iteration j (its own count, SB_ITER) writes ring
 // slot j % w and reads slot (j - 1) % w: the direction carries over the
 // steps a system sits out and its residual replacements.
-template <int ND, int TR, int TC>
-__global__ void __launch_bounds__(TR *TC + (TILE_HALO ? 64 : 0)) k_apply_dir(const Sys *__restrict__ sys, const Tile *__restrict__ tiles,
+template <int ND, int TR, int TC, bool HALO>
+__global__ void __launch_bounds__(TR *TC + (HALO ? 64 : 0)) k_apply_dir(const Sys *__restrict__ sys, const Tile *__restrict__ tiles,
                                                        const float *z, float *ring, size_t total, int w, float *q,
                                                        const double *__restrict__ Sb, double *__restrict__ part)
 {
@@ -86,7 +86,7 @@ __global__ void __launch_bounds__(TR *TC + (TILE_HALO ? 64 : 0)) k_apply_dir(con
     fz.dnew = ring + (size_t)(j % uw) * total + S.off;
     fz.first = R[SB_FRESH] != 0.0 ? 1 : 0;
     fz.beta = fz.first ? 0.f : (float)(R[SB_DELTA] / R[SB_DELTA_OLD]);
-    const double d = walsh_tile<float, ND, TR, TC, true, 1, TILE_HALO>(dold + S.off, q + S.off, S.keys, (const float *)S.mat32, 0,
+    const double d = walsh_tile<float, ND, TR, TC, true, 1, HALO>(dold + S.off, q + S.off, S.keys, (const float *)S.mat32, 0,
                                                             S.ny, S.nx, S.nz, S.LZ, t.bx, t.by, t.bz, fz).dq;
     const double s = bsum(d);
     if (threadIdx.x == 0) part[t.slot] = s;
@@ -94,8 +94,8 @@ __global__ void __launch_bounds__(TR *TC + (TILE_HALO ? 64 : 0)) k_apply_dir(con
 
 // Single-kernel step of the z-form loop (see apply_cg1 in batch.h); 4
 // partials per tile at part[k * ntiles + tile].
-template <int ND, int TR, int TC>
-__global__ void __launch_bounds__(TR *TC + (TILE_HALO ? 64 : 0)) k_apply_cg1(const Sys *__restrict__ sys, const Tile *__restrict__ tiles,
+template <int ND, int TR, int TC, bool HALO>
+__global__ void __launch_bounds__(TR *TC + (HALO ? 64 : 0)) k_apply_cg1(const Sys *__restrict__ sys, const Tile *__restrict__ tiles,
                                                        int ntiles, float *z1, float *z2, float *q1, float *q2,
                                                        float *ring, size_t total, int w,
                                                        const double *__restrict__ Sb, double *__restrict__ part)
@@ -125,7 +125,7 @@ __global__ void __launch_bounds__(TR *TC + (TILE_HALO ? 64 : 0)) k_apply_cg1(con
     fz.zring = zr ? 1 : 0;
     fz.bprev = zr ? (float)R[SB_BPREV] : 0.f;
     fz.lean = 0;
-    const TileSums ts = walsh_tile<float, ND, TR, TC, true, 2, TILE_HALO>(dold, qb[j & 1], S.keys, (const float *)S.mat32, 0,
+    const TileSums ts = walsh_tile<float, ND, TR, TC, true, 2, HALO>(dold, qb[j & 1], S.keys, (const float *)S.mat32, 0,
                                                              S.ny, S.nx, S.nz, S.LZ, t.bx, t.by, t.bz, fz);
     double v[4] = {ts.dq, ts.zq, ts.qmq, ts.zdz};
     block_sum<4>(v);
@@ -481,14 +481,33 @@ __global__ void __launch_bounds__(BB) k_resid_z(const Sys *__restrict__ sys, con
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
+// KERNEL for the batch's tile shape and values per node
+#define BATCH_GO(KERNEL_ND, NT, ARGS) KERNEL_ND<<<b.ntiles, NT, 0, s>>> ARGS
+#define BATCH_SHAPES(KERNEL, ARGS)                                                     \
+    if (b.nd == 3) {                                                                   \
+        if (b.shape == 1) BATCH_GO((KERNEL<3, 32, 8, false>), 256, ARGS);              \
+        else if (b.shape == 2) BATCH_GO((KERNEL<3, 64, 8, false>), 512, ARGS);         \
+        else BATCH_GO((KERNEL<3, 64, 7, true>), 512, ARGS);                            \
+    } else {                                                                           \
+        if (b.shape == 1) BATCH_GO((KERNEL<1, 32, 8, false>), 256, ARGS);              \
+        else if (b.shape == 2) BATCH_GO((KERNEL<1, 64, 8, false>), 512, ARGS);         \
+        else BATCH_GO((KERNEL<1, 64, 7, true>), 512, ARGS);                            \
+    }
+#define BATCH_SHAPES_T(KERNEL, ARGS)                                                   \
+    if (b.nd == 3) {                                                                   \
+        if (b.shape == 1) BATCH_GO((KERNEL<T, 3, 32, 8, false>), 256, ARGS);           \
+        else if (b.shape == 2) BATCH_GO((KERNEL<T, 3, 64, 8, false>), 512, ARGS);      \
+        else BATCH_GO((KERNEL<T, 3, 64, 7, true>), 512, ARGS);                         \
+    } else {                                                                           \
+        if (b.shape == 1) BATCH_GO((KERNEL<T, 1, 32, 8, false>), 256, ARGS);           \
+        else if (b.shape == 2) BATCH_GO((KERNEL<T, 1, 64, 8, false>), 512, ARGS);      \
+        else BATCH_GO((KERNEL<T, 1, 64, 7, true>), 512, ARGS);                         \
+    }
 template <typename T>
 void apply(const Batch &b, const T *v, T *q, int mode, hipStream_t s)
 {
     if (b.ntiles == 0) return;
-    if (b.nd == 3)
-        k_apply_walsh<T, 3, TILE_R, TILE_C><<<b.ntiles, TILE_THREADS, 0, s>>>(b.sys, b.tiles, v, q, b.Sb, b.part, mode);
-    else
-        k_apply_walsh<T, 1, TILE_R, TILE_C><<<b.ntiles, TILE_THREADS, 0, s>>>(b.sys, b.tiles, v, q, b.Sb, b.part, mode);
+    BATCH_SHAPES_T(k_apply_walsh, (b.sys, b.tiles, v, q, b.Sb, b.part, mode))
 }
 template void apply<float>(const Batch &, const float *, float *, int, hipStream_t);
 template void apply<double>(const Batch &, const double *, double *, int, hipStream_t);
@@ -506,12 +525,7 @@ void finish_alpha(const Batch &b, int w, hipStream_t s)
 void apply_dir(const Batch &b, const float *z, float *ring, size_t total, int w, float *q, hipStream_t s)
 {
     if (b.ntiles == 0) return;
-    if (b.nd == 3)
-        k_apply_dir<3, TILE_R, TILE_C><<<b.ntiles, TILE_THREADS, 0, s>>>(b.sys, b.tiles, z, ring, total, w, q, b.Sb,
-                                                                          b.part);
-    else
-        k_apply_dir<1, TILE_R, TILE_C><<<b.ntiles, TILE_THREADS, 0, s>>>(b.sys, b.tiles, z, ring, total, w, q, b.Sb,
-                                                                          b.part);
+    BATCH_SHAPES(k_apply_dir, (b.sys, b.tiles, z, ring, total, w, q, b.Sb, b.part))
 }
 
 void zupdate(const Batch &b, float *z, const float *q, hipStream_t s)
@@ -540,12 +554,7 @@ void apply_cg1(const Batch &b, float *z, float *z2, float *q, float *q2, float *
                hipStream_t s)
 {
     if (b.ntiles == 0) return;
-    if (b.nd == 3)
-        k_apply_cg1<3, TILE_R, TILE_C><<<b.ntiles, TILE_THREADS, 0, s>>>(b.sys, b.tiles, b.ntiles, z, z2, q, q2, ring,
-                                                                           total, w, b.Sb, b.part);
-    else
-        k_apply_cg1<1, TILE_R, TILE_C><<<b.ntiles, TILE_THREADS, 0, s>>>(b.sys, b.tiles, b.ntiles, z, z2, q, q2, ring,
-                                                                           total, w, b.Sb, b.part);
+    BATCH_SHAPES(k_apply_cg1, (b.sys, b.tiles, b.ntiles, z, z2, q, q2, ring, total, w, b.Sb, b.part))
     k_finish_cg1<<<b.nsys, BB, 0, s>>>(b.sys, b.Sb, b.part, b.ntiles, w);
 }
 

@@ -1816,13 +1816,18 @@ int chfemBatchSolve(void *h, double tol, unsigned int maxit)
     std::vector<Chunk> chunks;
     std::vector<std::pair<int, int>> owner;  // (sample, load) of each system
     size_t off = 0;
+    std::vector<std::array<int, 3>> dims;
+    for (const BatchSample &bs : B->samples) dims.push_back({(int)bs.m->ey, (int)bs.m->ex, (int)bs.m->ez});
+    int lz = 16;
+    const int shape = batch_tile_rule(nd == 3, SHAPES, NSHAPES, dims, nloads, lz);
+    const Shape tile = SHAPES[shape];
     for (size_t si = 0; si < B->samples.size(); si++) {
         const Model &m = *B->samples[si].m;
         for (int d = 0; d < nloads; d++) {
             Sys S;
             memset(&S, 0, sizeof(S));
             S.ny = (int)m.ey; S.nx = (int)m.ex; S.nz = (int)m.ez;
-            S.LZ = TILE_LZ;
+            S.LZ = lz;
             S.N = (uint32_t)m.nelem;
             S.off = off;
             S.keys = B->samples[si].keys;
@@ -1831,7 +1836,7 @@ int chfemBatchSolve(void *h, double tol, unsigned int maxit)
             const int sid = (int)sys.size();
             S.tb0 = (int)tiles.size();
             {
-                const int gx = (S.ny + TILE_ROWS - 1) / TILE_ROWS, gy = (S.nx + TILE_C - 2) / (TILE_C - 1);
+                const int gx = (S.ny + tile.rows - 1) / tile.rows, gy = (S.nx + tile.cols - 1) / tile.cols;
                 const int gz = (S.nz + S.LZ - 1) / S.LZ;
                 for (int z = 0; z < gz; z++)
                     for (int y = 0; y < gy; y++)
@@ -1899,7 +1904,7 @@ int chfemBatchSolve(void *h, double tol, unsigned int maxit)
         }
     }
     Batch bt;
-    bt.nsys = nsys; bt.nd = nd; bt.sys = dsys; bt.tiles = dtiles; bt.ntiles = (int)tiles.size();
+    bt.nsys = nsys; bt.nd = nd; bt.shape = shape; bt.sys = dsys; bt.tiles = dtiles; bt.ntiles = (int)tiles.size();
     bt.chunks = dchunks; bt.nchunks = (int)chunks.size(); bt.Sb = Sb; bt.part = part;
     std::vector<double> Sh((size_t)nsys * SB_STRIDE, 0.0);
     auto down = [&]() {

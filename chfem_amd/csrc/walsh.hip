@@ -6,6 +6,7 @@
 
 #include <algorithm>
 
+#include "batch.h"
 #include "walsh.h"
 
 namespace chfem {
@@ -221,27 +222,77 @@ template void launch_walsh_lean<double>(const OpDesc &, int, const double *, dou
 // every tile and LZ 1 to 32.  Over those grids the pick is within 3 % of the
 // fastest candidate, 10 % at the worst, where timing every candidate before
 // the first solve cost as much as 30 (256^3) to 150 (32^3) iterations.
-template <typename T>
-static double tile_cost(const OpDesc &op, int tr, int tc, int lz)
+struct TileFit {
+    double L, c, d, h;  // see above
+    int resident;       // blocks resident on a CU
+    double step(double on_cu, int nt) const { return d + std::max(L, on_cu * nt * c); }
+};
+
+static TileFit tile_fit(bool dbl, bool el, int nt)
 {
-    const bool dbl = sizeof(T) == 8, el = op.physics == PHY_ELASTIC;
     static const double fit[2][2][4] = {  // [precision][physics] L, c, d, h
         {{0.400, 0.00059, 0.337, 1.345}, {0.380, 0.00091, 0.699, 4.266}},
         {{0.839, 0.00134, 0.000, 1.692}, {0.482, 0.00268, 0.920, 4.836}}};
     // blocks of 256 and of 512 work-items resident on a CU
     static const int resident[2][2][2] = {{{8, 4}, {5, 2}}, {{6, 3}, {3, 1}}};
     const double *f = fit[dbl][el];
-    const bool halo = tr == 65;
+    return {f[0], f[1], f[2], f[3], resident[dbl][el][nt > 256]};
+}
+
+template <typename T>
+static double tile_cost(const OpDesc &op, int tr, int tc, int lz)
+{
+    const bool el = op.physics == PHY_ELASTIC, halo = tr == 65;
     const int owned = halo ? 64 : tr - 1, nt = halo ? 64 * tc + 64 : tr * tc;
-    const int per_cu = resident[dbl][el][nt > 256];
+    const TileFit f = tile_fit(sizeof(T) == 8, el, nt);
     const double nb = (double)((op.ny + owned - 1) / owned) * ((op.nx + tc - 2) / (tc - 1)) * ((op.nz + lz - 1) / lz);
-    auto step = [&](double on_cu) { return f[2] + std::max(f[0], on_cu * nt * f[1]); };
-    const double slots = 256.0 * per_cu, full = floor(nb / slots), rest = nb - full * slots;
+    const double slots = 256.0 * f.resident, full = floor(nb / slots), rest = nb - full * slots;
     const double steps = std::min(lz, op.nz) + 2;
-    const double chain = full * step(per_cu) + (rest > 0 ? step(ceil(rest / 256.0)) : 0.0);
+    const double chain = full * f.step(f.resident, nt) + (rest > 0 ? f.step(ceil(rest / 256.0), nt) : 0.0);
     const double vb = sizeof(T) * (el ? 3 : 1);
     const double loaded = nb * (tc + 1) * ((owned + 2) + 128.0 / vb) * steps * 1e-6;
-    return chain * steps + f[3] * loaded;
+    return chain * steps + f.h * loaded;
+}
+
+// The same cost for a batch (FP32), summed over its samples: rounds of blocks
+// become the layer steps of all blocks over the resident slots.  At most 16
+// layers per block: with 32 the last blocks of an uneven batch run alone (8
+// samples of edges 48-80, elastic: 195 ms against 179 with 16).  That batch
+// took 217 ms on 64 x 7 tiles of 32 layers (two row tiles for 65-80 rows);
+// picked: 32 x 8 x 16.  4 samples of edges 20-32: 23.7 -> 10.1 ms (32 x 8 x 4);
+// 3 of 90-130: 515 -> 454 (32 x 8 x 16); 6 of 60-66: 146 -> 135 (64 x 7 x 16);
+// thermal, 8 of 48-80: 28.2 -> 23.8 (64 x 8 x 16; 21.7 with 32 x 8 x 8).
+int batch_tile_rule(bool elastic, const batch::Shape *shapes, int nshapes, const std::vector<std::array<int, 3>> &dims,
+                    int loads, int &lz_out)
+{
+    int best = 0;
+    double least = 1e300;
+    for (int sh = 0; sh < nshapes; sh++) {
+        const batch::Shape &t = shapes[sh];
+        const int nt = t.tr == 65 ? 64 * t.tc + 64 : t.tr * t.tc;
+        const TileFit f = tile_fit(false, elastic, nt);
+        const double vb = sizeof(float) * (elastic ? 3 : 1);
+        for (int lz = 1; lz <= 16; lz *= 2) {
+            double nb = 0, steps = 0, longest = 0;
+            for (const auto &n : dims) {  // {ny, nx, nz}
+                const double cols = (double)((n[0] + t.rows - 1) / t.rows) * ((n[1] + t.cols - 1) / t.cols) * loads;
+                const int chunks = (n[2] + lz - 1) / lz;
+                nb += cols * chunks;
+                steps += cols * (n[2] + 2 * chunks);
+                longest = std::max(longest, std::min(lz, n[2]) + 2.0);
+            }
+            const double chain = longest * f.step(std::min((double)f.resident, ceil(nb / 256.0)), nt);
+            const double all = steps / (256.0 * f.resident) * f.step(f.resident, nt);
+            const double cost = std::max(chain, nb >= 256.0 * f.resident ? all : 0.0) +
+                                f.h * steps * (t.tc + 1) * ((t.rows + 2) + 128.0 / vb) * 1e-6;
+            if (cost < least) {
+                least = cost;
+                best = sh;
+                lz_out = lz;
+            }
+        }
+    }
+    return best;
 }
 
 template <typename T>

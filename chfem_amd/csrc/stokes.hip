@@ -160,11 +160,19 @@ __device__ __forceinline__ void lean_dof(const StokesLean<T> &L, T u, T o, T inv
     }
 }
 
+constexpr int STOKES_LZ = 16;  // node layers per block, unless told otherwise
+
 // One tile of the Stokes operator (see walsh_tile for the march, the tile
 // order and the load pipelining; here a plane node holds (u, v, w, p)
 // gathered through the node-to-DOF map, whose entries and keys are loaded
 // one layer ahead of the value gathers).
-template <typename T, int TR, int TC, bool DOT, bool LEAN = false>
+//
+// NG groups of TR * TC work-items march LZ / NG layers each of one block, for
+// grids that leave the chip idle.  MINRES amplifies a change of rounding (its
+// pressure preconditioner is indefinite), so the dot's partial sums keep their
+// order: the groups keep each layer's products and add them one group after
+// the other, layer by layer, as one group does.
+template <typename T, int TR, int TC, int NG, bool DOT, bool LEAN = false>
 __device__ __forceinline__ double stokes_tile(const T *__restrict__ v, T *__restrict__ q,
                                               const uint32_t *__restrict__ node2dof, const uint8_t *__restrict__ fk,
                                               uint32_t nvel, int ny, int nx, int nz, int LZ, int bx, int by, int bz,
@@ -174,12 +182,20 @@ __device__ __forceinline__ double stokes_tile(const T *__restrict__ v, T *__rest
     constexpr int NS = (NN + NT - 1) / NT;  // plane nodes per work-item
     constexpr int SB = 9;                   // 2 x 4 row-combined forces + pad
     static_assert(TR == 16 || TR == 32 || TR == 64, "rows per tile must tile a 64-wide wavefront");
-    __shared__ __align__(16) T su[2][NS * NT * 4];
-    __shared__ T sb[NT * SB];
-    const int tid = threadIdx.x;
+    constexpr int G = STOKES_LZ / NG;       // most layers per group (NG > 1)
+    static_assert(NG == 1 || (DOT && !LEAN), "layer groups are for the operator with its dot");
+    __shared__ __align__(16) T su_[NG][2][NS * NT * 4];
+    __shared__ T sb_[NG][NT * SB];
+    const int grp = NG > 1 ? (int)threadIdx.x / NT : 0, tid = (int)threadIdx.x - grp * NT;
+    T(&su)[2][NS * NT * 4] = su_[grp];
+    T *sb = sb_[grp];
     const int tr = tid % TR, tc = tid / TR;
-    const int r0 = bx * (TR - 1), c0 = by * (TC - 1), l0 = bz * LZ;
-    const int vr = min(TR - 1, ny - r0), vc = min(TC - 1, nx - c0), vl = min(LZ, nz - l0);
+    const int r0 = bx * (TR - 1), c0 = by * (TC - 1);
+    const int gl = NG > 1 ? (min(LZ, nz - bz * LZ) + NG - 1) / NG : LZ;  // layers per group of this block
+    const int l0 = bz * LZ + grp * gl;
+    // (a group whose layers lie past the last one has vl <= 0: it marches with
+    // the others, on wrapped layers, and owns nothing)
+    const int vr = min(TR - 1, ny - r0), vc = min(TC - 1, nx - c0), vl = min(gl, nz - l0);
     const size_t nxy = (size_t)nx * ny;
     const T *vp = v + 3 * (size_t)nvel;  // pressures
     auto wrapl = [&](int lg) {
@@ -291,7 +307,8 @@ __device__ __forceinline__ double stokes_tile(const T *__restrict__ v, T *__rest
     bool pe = is_pore(ek);
     ek = elem_key(l0);
     // owned node's DOF id and key, one layer ahead
-    uint32_t oid = node2dof[(size_t)l0 * nxy + own_off], okey = fk[(size_t)l0 * nxy + own_off];
+    const size_t first = (size_t)(NG > 1 ? wrapl(l0) : l0) * nxy;
+    uint32_t oid = node2dof[first + own_off], okey = fk[first + own_off];
     __syncthreads();
     fetch(l0 + 1);
     T A[4], Af[4];
@@ -307,7 +324,11 @@ __device__ __forceinline__ double stokes_tile(const T *__restrict__ v, T *__rest
     }
     __syncthreads();
     double dsum = 0.0;
-    for (int s = 0; s < vl; s++) {
+    double hist[G][3];  // NG > 1: the layers' products, oldest first (zeros before them)
+#pragma unroll
+    for (int k = 0; k < G; k++) hist[k][0] = hist[k][1] = hist[k][2] = 0.0;
+    const int steps = NG > 1 ? gl : vl;
+    for (int s = 0; s < steps; s++) {
         const int l = l0 + s;
         const uint32_t id = oid, key = okey;
         oid = node2dof[(size_t)wrapl(l + 1) * nxy + own_off];
@@ -320,7 +341,16 @@ __device__ __forceinline__ double stokes_tile(const T *__restrict__ v, T *__rest
         __syncthreads();
         store(cur);  // layer l + 2 replaces layer l
         pe = is_pore(ek);
-        if (own) {
+        if constexpr (NG > 1) {
+#pragma unroll
+            for (int k = 0; k + 1 < G; k++) {
+                hist[k][0] = hist[k + 1][0];
+                hist[k][1] = hist[k + 1][1];
+                hist[k][2] = hist[k + 1][2];
+            }
+            hist[G - 1][0] = hist[G - 1][1] = hist[G - 1][2] = 0.0;
+        }
+        if (own && (NG == 1 || s < vl)) {
             T o[4];
 #pragma unroll
             for (int a = 0; a < 4; a++) {
@@ -341,11 +371,20 @@ __device__ __forceinline__ double stokes_tile(const T *__restrict__ v, T *__rest
                 if (key == 255u) {
                     T *qo = q + 3 * (size_t)id;
                     qo[0] = o[0]; qo[1] = o[1]; qo[2] = o[2];
-                    if (DOT) dsum += (double)own_u[0] * o[0] + (double)own_u[1] * o[1] + (double)own_u[2] * o[2];
+                    if (DOT) {
+                        const double d = (double)own_u[0] * o[0] + (double)own_u[1] * o[1] + (double)own_u[2] * o[2];
+                        if (NG > 1) hist[G - 1][0] = d;
+                        else dsum += d;
+                    }
                 }
                 if (key != 0u) {
                     q[3 * (size_t)nvel + id] = o[3];
-                    if (DOT) dsum += (double)own_u[3] * o[3];
+                    if (NG > 1) {
+                        hist[G - 1][1] = (double)own_u[3];
+                        hist[G - 1][2] = (double)o[3];
+                    } else if (DOT) {
+                        dsum += (double)own_u[3] * o[3];
+                    }
                 }
             }
         }
@@ -354,11 +393,27 @@ __device__ __forceinline__ double stokes_tile(const T *__restrict__ v, T *__rest
         }
         __syncthreads();
     }
+    if constexpr (NG > 1) {
+        __shared__ double chain[NT];
+        for (int g = 0; g < NG; g++) {
+            if (grp == g) {
+                if (g > 0) dsum = chain[tid];
+#pragma unroll
+                for (int k = 0; k < G; k++) {
+                    dsum += hist[k][0];
+                    dsum += hist[k][1] * hist[k][2];
+                }
+                chain[tid] = dsum;
+            }
+            __syncthreads();
+        }
+        if (grp != NG - 1) dsum = 0.0;
+    }
     return dsum;
 }
 
-template <typename T, int TR, int TC, bool DOT, bool LEAN = false>
-__global__ void __launch_bounds__(TR *TC) k_stokes_walsh(const T *__restrict__ v, T *__restrict__ q,
+template <typename T, int TR, int TC, int NG, bool DOT, bool LEAN = false>
+__global__ void __launch_bounds__(TR *TC *NG) k_stokes_walsh(const T *__restrict__ v, T *__restrict__ q,
                                                           const uint32_t *__restrict__ node2dof,
                                                           const uint8_t *__restrict__ fk, uint32_t nvel, int ny, int nx,
                                                           int nz, int LZ, Reduce red,
@@ -370,7 +425,7 @@ __global__ void __launch_bounds__(TR *TC) k_stokes_walsh(const T *__restrict__ v
     const unsigned gx = (unsigned)(ny + TR - 2) / (TR - 1), gy = (unsigned)(nx + TC - 2) / (TC - 1);
     const unsigned b = blockIdx.x, nb = gridDim.x, per = nb / 8u, rem = nb % 8u, xcd = b % 8u, k = b / 8u;
     const unsigned t = (xcd < rem ? xcd * (per + 1u) : rem * (per + 1u) + (xcd - rem) * per) + k;
-    const double dsum = stokes_tile<T, TR, TC, DOT, LEAN>(v, q, node2dof, fk, nvel, ny, nx, nz, LZ, (int)(t % gx),
+    const double dsum = stokes_tile<T, TR, TC, NG, DOT, LEAN>(v, q, node2dof, fk, nvel, ny, nx, nz, LZ, (int)(t % gx),
                                                           (int)((t / gx) % gy), (int)(t / (gx * gy)), L);
     if (DOT) {
         double vv[1] = {dsum};
@@ -391,16 +446,26 @@ void launch_stokes_walsh(const OpDesc &op, const T *v, T *q, const Reduce *red, 
     Reduce rr = {nullptr, nullptr, 0, 0, 0};
     if (red) rr = *red;
     constexpr int TR = 32, TC = 8;
-    int LZ = op.tile_lz > 0 ? op.tile_lz : 16;
+    int LZ = op.tile_lz > 0 ? op.tile_lz : STOKES_LZ;
     const long cols = (long)((op.ny + TR - 2) / (TR - 1)) * ((op.nx + TC - 2) / (TC - 1));
     while (cols * ((op.nz + LZ - 1) / LZ) > MAX_PARTIAL_BLOCKS) LZ *= 2;
     const unsigned grid = (unsigned)cols * (unsigned)((op.nz + LZ - 1) / LZ);
-    if (red) {
-        k_stokes_walsh<T, TR, TC, true><<<grid, TR * TC, 0, s>>>(v, q, op.node2dof, op.fkeys, op.nvel, op.ny, op.nx,
+    if (red && LZ == STOKES_LZ && grid <= 256) {
+        // At most one block per CU: the time is the march of one block, whose
+        // FP64 arithmetic a wavefront issues alone on its SIMD.  Two groups of
+        // half the layers: MINRES iterations of a 100x100x10 slab (60 blocks)
+        // 40.6 -> 37.2 us, 64^3 (120) 51.3 -> 45.8, 80^3 (180) 55.8 -> 50.0.
+        // With more blocks the CUs are shared anyway and each group's two
+        // extra layers count: 96^3 (336) 71.6 -> 78.7, 160^3 185 -> 233.
+        k_stokes_walsh<T, TR, TC, 2, true><<<grid, 2 * TR * TC, 0, s>>>(v, q, op.node2dof, op.fkeys, op.nvel, op.ny,
+                                                                        op.nx, op.nz, LZ, rr);
+        launch_reduce_finish(rr, grid, 1, s);
+    } else if (red) {
+        k_stokes_walsh<T, TR, TC, 1, true><<<grid, TR * TC, 0, s>>>(v, q, op.node2dof, op.fkeys, op.nvel, op.ny, op.nx,
                                                                  op.nz, LZ, rr);
         launch_reduce_finish(rr, grid, 1, s);
     } else {
-        k_stokes_walsh<T, TR, TC, false><<<grid, TR * TC, 0, s>>>(v, q, op.node2dof, op.fkeys, op.nvel, op.ny, op.nx,
+        k_stokes_walsh<T, TR, TC, 1, false><<<grid, TR * TC, 0, s>>>(v, q, op.node2dof, op.fkeys, op.nvel, op.ny, op.nx,
                                                                   op.nz, LZ, rr);
     }
 }
@@ -410,13 +475,13 @@ void launch_stokes_lean(const OpDesc &op, const Jac<T> &jac, int form, const T *
                         hipStream_t s)
 {
     constexpr int TR = 32, TC = 8;
-    int LZ = op.tile_lz > 0 ? op.tile_lz : 16;
+    int LZ = op.tile_lz > 0 ? op.tile_lz : STOKES_LZ;
     const long cols = (long)((op.ny + TR - 2) / (TR - 1)) * ((op.nx + TC - 2) / (TC - 1));
     while (cols * ((op.nz + LZ - 1) / LZ) > MAX_PARTIAL_BLOCKS) LZ *= 2;
     const unsigned grid = (unsigned)cols * (unsigned)((op.nz + LZ - 1) / LZ);
     const bool pc = jac.kind == JAC_FLUID;
     const StokesLean<T> L = {form, T(0), pc ? jac.vinv : T(1), pc ? jac.pinv : T(1), pc ? jac.btab : nullptr};
-    k_stokes_walsh<T, TR, TC, true, true><<<grid, TR * TC, 0, s>>>(v, z, op.node2dof, op.fkeys, op.nvel, op.ny, op.nx,
+    k_stokes_walsh<T, TR, TC, 1, true, true><<<grid, TR * TC, 0, s>>>(v, z, op.node2dof, op.fkeys, op.nvel, op.ny, op.nx,
                                                                    op.nz, LZ, *red, L);
     launch_reduce_finish(*red, grid, 1, s);
 }

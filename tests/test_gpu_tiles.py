@@ -99,3 +99,44 @@ def test_density_solves(shape, which, solver, precision):
         assert rel(m.update_c(0, x), m.update_c(0, xr)) < 1e-6
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("shape", [(2, 5, 9), (3, 33, 16), (7, 62, 30), (10, 100, 63), (16, 14, 31)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_stokes_layer_groups(shape, precision, monkeypatch):
+    """On grids of few tiles two groups of work-items share a tile's layers,
+    with the sums of one group: after 30 MINRES steps the solution has the same
+    bits as with one group (tiles of 32 layers: one chunk either way)."""
+    rng = np.random.default_rng(sum(shape))
+    img = np.where(rng.random(shape) < 0.3, 255, 0).astype(np.uint8)
+    img[:2, :2, :2] = 0  # the elements around one node: it is fully fluid
+    m = H.model(H.FLUID, img, [0.0], colors=(0, 255))
+    got = []
+    for tile in (None, "32x8x32"):
+        if tile:
+            monkeypatch.setenv("CHFEM_WALSH_TILE", tile)
+        s = H.GpuSolver(m, solver=1, precision=precision, tol=1e-30, maxit=30)
+        try:
+            x, _, st = s.solve(m.rhs(0))
+            got.append((x, st.iterations))
+        finally:
+            s.close()
+    assert got[0][1] == got[1][1] and np.abs(got[0][0]).max() > 0
+    assert np.array_equal(got[0][0], got[1][0])
+
+
+@pytest.mark.parametrize("nz", [17, 33])
+def test_stokes_layer_groups_solve(nz):
+    """Layer chunks shorter than a group: a whole solve against the oracle's."""
+    rng = np.random.default_rng(nz)
+    img = np.where(rng.random((nz, 20, 14)) < 0.1, 255, 0).astype(np.uint8)
+    m = H.model(H.FLUID, img, [0.0], colors=(0, 255))
+    s = H.GpuSolver(m, solver=1, tol=1e-9)
+    try:
+        x, ok, st = s.solve(m.rhs(2))
+        xr, okr, _, _ = m.solve(2, solver=1, tol=1e-9)
+        assert ok and okr
+        assert rel(m.update_c(2, x), m.update_c(2, xr)) < 1e-6
+    finally:
+        s.close()

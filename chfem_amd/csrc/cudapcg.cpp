@@ -158,6 +158,9 @@ Reduce make_reduce(int fin, int slot)
     r.guard = 0;
     r.partials2 = nullptr;
     r.nb2 = 0;
+    r.chain = r.defer = 0;
+    r.prev = r.Sin = nullptr;
+    r.Sout = nullptr;
     return r;
 }
 
@@ -357,7 +360,7 @@ static cudapcgFlag_t alloc_solver_arrays()
     }
     const size_t pn = (size_t)MAX_PARTIAL_BLOCKS * 8;
     if (!g->partials) CHECK_HIP(hipMalloc(&g->partials, pn * sizeof(double)));
-    if (!g->S) CHECK_HIP(hipMalloc(&g->S, S_COUNT * sizeof(double)));
+    if (!g->S) CHECK_HIP(hipMalloc(&g->S, S_ALLOC * sizeof(double)));
     if (!g->Sh) CHECK_HIP(hipHostMalloc((void **)&g->Sh, S_COUNT * sizeof(double), hipHostMallocDefault));
     CHECK_HIP(hipMemsetAsync(g->S, 0, S_COUNT * sizeof(double), g->stream));
     g->arrays = true;
@@ -772,6 +775,9 @@ static int run_pcg(const OpDesc &op, T *x, T *r, T *d, T *q, const T *dinv, bool
                     // the first writes z (the second reads it)
                     const bool zr = W >= 3 && j >= 2;
                     T *zw = W >= 3 && j >= 1 ? nullptr : zb[j & 1];
+                    // S is current again after the batch and before a flush
+                    rc.chain = rc.defer ? rc.chain + 1 : 0;
+                    rc.defer = b + 1 < nb && (j + 1) % W != 0 ? 1 : 0;
                     // (the timed launch: the third of the batch, a steady
                     // iteration)
                     timed_apply_cg1<T>(op, zb[(j + 1) & 1], qb[(j + 1) & 1], j > 0 ? slot(j - 1) : nullptr, zw,
@@ -1479,6 +1485,8 @@ static int run_mixed_reliable(bool x0set, unsigned &it_total, unsigned &sweeps, 
                         // segment's first iteration writes z
                         const bool zr = W >= 3 && j >= base + 2;
                         float *zw = W >= 3 && j >= base + 1 ? nullptr : zb[j & 1];
+                        rc.chain = rc.defer ? rc.chain + 1 : 0;
+                        rc.defer = b + 1 < nb && (j + 1) % W != 0 ? 1 : 0;
                         timed_apply_cg1<float>(o32, zb[(j + 1) & 1], qb[(j + 1) & 1], j > 0 ? slot(j - 1) : nullptr,
                                                zw, slot(j), qb[j & 1], j > base ? 1 : 0, &rc,
                                                b == (nb > 2 ? 2u : 0u), zr ? slot(j - 2) : nullptr);

@@ -26,7 +26,10 @@ enum ScalarSlot {
     S_BPREV,
     // alpha of guarded iteration j (j counted in S[S_ITER]) at
     // S[S_AHIST + j % S_AHIST_LEN], for the ring flush of the iterate
-    S_AHIST = 24, S_AHIST_LEN = 32, S_COUNT = S_AHIST + S_AHIST_LEN
+    S_AHIST = 24, S_AHIST_LEN = 32, S_COUNT = S_AHIST + S_AHIST_LEN,
+    // the scalars that odd iterations of a chain work on (Reduce::chain) start
+    // here; the slots below S_AHIST are used
+    S_CHAIN = S_COUNT, S_ALLOC = S_CHAIN + S_AHIST
 };
 
 // How the finishing kernel of a fused reduction publishes its total.
@@ -63,7 +66,19 @@ struct Reduce {
     // FIN_STOP_DELTA: the partials an earlier launch left (one value each)
     const double *partials2;
     unsigned nb2;
+    // Chained FIN_CG1 (launch_apply_cg1, small grids): the iterations between
+    // two points where S has to be current do without the finishing launch;
+    // each block of the next iteration adds the partials itself.  chain: the
+    // iterations queued since S was current (0: none); defer: the next
+    // iteration of this chain finishes this one.
+    int chain, defer;
+    // set by the launcher: the previous iteration's partials (null: S is
+    // current) and scalars, and where this launch leaves the scalars it read
+    const double *prev, *Sin;
+    double *Sout;
 };
+// blocks up to which iterations are chained (walsh.hip)
+#define CHAIN_BLOCKS 256
 
 // Scalar density field (EBE only): element e's local matrices are scaled by
 // d[e] * (1/65535) * (fmax - fmin) + fmin (chfem/src/femhmg/femhmg.c:1760-1835);

@@ -1177,7 +1177,7 @@ static inline int stream_grid(size_t n, size_t elem_bytes)
     return b < 1 ? 1 : (int)b;
 }
 
-static Reduce noreduce() { Reduce r; r.partials = nullptr; r.S = nullptr; r.fin = 0; r.slot = 0; r.guard = 0; r.partials2 = nullptr; r.nb2 = 0; return r; }
+static Reduce noreduce() { Reduce r; r.partials = nullptr; r.S = nullptr; r.fin = 0; r.slot = 0; r.guard = 0; r.partials2 = nullptr; r.nb2 = 0; r.chain = r.defer = 0; r.prev = r.Sin = nullptr; r.Sout = nullptr; return r; }
 
 // One block, bound by latency alone: the partials were written by all XCDs,
 // so every read misses this XCD's L2 (about 0.8 us).  The 16 wavefronts share
@@ -1193,9 +1193,10 @@ __global__ void __launch_bounds__(1024) k_reduce_finish(Reduce red, unsigned nb)
     constexpr int TURN = 8;
     __shared__ double part[WAVES], part2[WAVES];
     double *S = red.S;
+    const double *in = NV == 4 && red.Sin ? red.Sin : S;  // the end of a chain (Reduce::chain)
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, k = w / PER;
-    const double done = red.guard ? S[S_DONE] : 0.0;
-    const double delta_cur = S[S_DELTA], delta_old = S[S_DELTA_OLD], iter = S[S_ITER], thresh = S[S_THRESH];
+    const double done = red.guard ? in[S_DONE] : 0.0;
+    const double delta_cur = in[S_DELTA], delta_old = in[S_DELTA_OLD], iter = in[S_ITER], thresh = S[S_THRESH];
     auto list_sum = [&](const double *p, unsigned nb) -> double {
         double sum = 0;
         for (unsigned b0 = (w % PER) * 64 + lane; b0 < nb; b0 += PER * 64 * TURN) {
@@ -1219,7 +1220,11 @@ __global__ void __launch_bounds__(1024) k_reduce_finish(Reduce red, unsigned nb)
         if (lane == 0) part2[w] = sum;
     }
     __syncthreads();
-    if (threadIdx.x != 0 || done != 0.0) return;
+    if (threadIdx.x != 0) return;
+    if (done != 0.0) {
+        if (in != S) cg1_store(S, cg1_load(in));
+        return;
+    }
     double s[NV];
 #pragma unroll
     for (int v = 0; v < NV; v++) {
@@ -1240,23 +1245,17 @@ __global__ void __launch_bounds__(1024) k_reduce_finish(Reduce red, unsigned nb)
             if (fabs(s[0]) <= thresh) S[S_DONE] = 1.0;
         }
     } else if (red.fin == FIN_CG1 && NV == 4) {
-        // delta of this iteration from its own z (s[3]), not carried
-        // over from the previous recurrence step: rounding then reaches
-        // beta through one step only
-        const double delta = s[3 % NV], alpha = delta / s[0];
-        const double dnew = delta - 2.0 * alpha * s[1 % NV] + alpha * alpha * s[2 % NV];
-        // the beta this iteration's launch formed its direction with
-        // (the same quotient it computed), for the next launch that
-        // recovers z from the directions
-        S[S_BPREV] = delta_cur / delta_old;
+        const Cg1Scalars c = cg1_finish(s[0], s[1 % NV], s[2 % NV], s[3 % NV], delta_cur, delta_old, iter,
+                                        red.guard ? thresh : -1.0);
         S[S_DQ] = s[0];
-        S[S_ALPHA] = alpha;
-        S[S_DELTA_OLD] = delta;
-        S[S_DELTA] = dnew;
+        S[S_BPREV] = c.bprev;
+        S[S_ALPHA] = c.alpha;
+        S[S_DELTA_OLD] = c.delta_old;
+        S[S_DELTA] = c.delta;
         if (red.guard) {
-            S[S_AHIST + (unsigned)iter % S_AHIST_LEN] = alpha;
-            S[S_ITER] = iter + 1.0;
-            if (fabs(dnew) <= thresh) S[S_DONE] = 1.0;
+            S[S_AHIST + (unsigned)iter % S_AHIST_LEN] = c.alpha;
+            S[S_ITER] = c.iter;
+            S[S_DONE] = c.done;
         }
     } else if (red.fin == FIN_STOP) {
         S[S_STOP] = s[0];

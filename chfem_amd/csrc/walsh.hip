@@ -11,6 +11,16 @@
 
 namespace chfem {
 
+__device__ __forceinline__ float wave_uniform(float v)
+{
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
+}
+__device__ __forceinline__ double wave_uniform(double v)
+{
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
 template <typename T, int ND, int TR, int TC, bool DOT, int FM, bool HALO, bool SDF>
 __device__ __forceinline__ void walsh_block(const T *__restrict__ v, T *__restrict__ q,
                                             const uint16_t *__restrict__ keys, const T *__restrict__ lamu, int ebe,
@@ -19,20 +29,36 @@ __device__ __forceinline__ void walsh_block(const T *__restrict__ v, T *__restri
     constexpr bool FUSE = FM == 1 || FM == 2;
     // the scalars are read together, before the stop flag is tested: one
     // read latency at the head of the launch instead of two
-    const double done = DOT && red.guard ? red.S[S_DONE] : 0.0;
-    double iter = 0.0;
-    // beta of the fused direction update, as k_kj_pcg_dir forms it
-    if (FUSE && !fz.first) fz.beta = (T)(red.S[S_DELTA] / red.S[S_DELTA_OLD]);
-    // single-kernel CG: alpha of the previous iteration for the deferred z
-    // update
-    if (FM == 2) fz.alpha = fz.zpend ? (T)red.S[S_ALPHA] : T(0);
-    // single-kernel CG with z recovered from the ring: the beta that formed
-    // d_old
-    if (FM == 2 && fz.zring) fz.bprev = (T)red.S[S_BPREV];
-    // lean z update: alpha of this iteration
-    if (FM == 3) fz.alpha = fz.lean == LEAN_ZUPD ? (T)red.S[S_ALPHA] : T(0);
-    if (FM == 2 && DOT && red.guard) iter = red.S[S_ITER];
+    double done = 0.0, iter = 0.0;
+    if (FM == 2 && DOT && red.prev) {
+        const Cg1Scalars c = cg1_chain(red, gridDim.x);
+        if (c.done != 0.0) return;
+        fz.beta = (T)(c.delta / c.delta_old);
+        fz.alpha = fz.zpend ? (T)c.alpha : T(0);
+        if (fz.zring) fz.bprev = (T)c.bprev;
+        iter = c.iter;
+    } else {
+        done = DOT && red.guard ? red.S[S_DONE] : 0.0;
+        // beta of the fused direction update, as k_kj_pcg_dir forms it
+        if (FUSE && !fz.first) fz.beta = (T)(red.S[S_DELTA] / red.S[S_DELTA_OLD]);
+        // single-kernel CG: alpha of the previous iteration for the deferred z
+        // update
+        if (FM == 2) fz.alpha = fz.zpend ? (T)red.S[S_ALPHA] : T(0);
+        // single-kernel CG with z recovered from the ring: the beta that formed
+        // d_old
+        if (FM == 2 && fz.zring) fz.bprev = (T)red.S[S_BPREV];
+        // lean z update: alpha of this iteration
+        if (FM == 3) fz.alpha = fz.lean == LEAN_ZUPD ? (T)red.S[S_ALPHA] : T(0);
+        if (FM == 2 && DOT && red.guard) iter = red.S[S_ITER];
+    }
     if (done != 0.0) return;
+    if (FM == 2) {
+        // the same in every lane: kept in scalar registers (with them in
+        // vector registers the FP64 thermal tiles lose a wavefront per SIMD)
+        fz.beta = wave_uniform(fz.beta);
+        fz.alpha = wave_uniform(fz.alpha);
+        fz.bprev = wave_uniform(fz.bprev);
+    }
     // 1-D grid; blocks are dispatched to the 8 XCDs round-robin (block b to
     // XCD b % 8), so each XCD is given one contiguous range of tiles (rows of
     // tiles fastest): tiles that share halo nodes then run on the same XCD at
@@ -77,6 +103,30 @@ __global__ void __launch_bounds__(TR *TC + (HALO ? 64 : 0)) k_walsh_sdf(const T 
     walsh_block<T, ND, TR, TC, DOT, FM, HALO, true>(v, q, elems, lamu, 1, ny, nx, nz, LZ, red, fz);
 }
 
+// Chained iterations (Reduce::chain): even ones work on S, odd ones on the
+// scalars and partials kept beside them.  Sets this launch's inputs in rr and
+// returns the Reduce of its finishing kernel, which is launched unless
+// rr.defer.  On grids of one block per CU or less an iteration is little but
+// latency: without the finishing launch, CG iterations take 24^3 thermal FP64
+// 11.2 -> 10.0 us, 32^3 11.9 -> 11.3, 32^3 elastic 14.9 -> 13.8, 64^3 23.7 ->
+// 22.7.  With more blocks each would read more partials than the one
+// finishing block saves.
+static Reduce cg1_plan(Reduce &rr, unsigned grid)
+{
+    if (!rr.guard || grid > CHAIN_BLOCKS) rr.chain = rr.defer = 0;
+    double *const P[2] = {rr.partials, rr.partials + 4 * CHAIN_BLOCKS}, *const S[2] = {rr.S, rr.S + S_CHAIN};
+    const int odd = rr.chain & 1;
+    if (rr.chain) {
+        rr.prev = P[odd ^ 1];
+        rr.Sin = S[odd ^ 1];
+        rr.Sout = S[odd];
+    }
+    rr.partials = P[odd];
+    Reduce fin = rr;
+    fin.Sin = S[odd];
+    return fin;
+}
+
 template <typename T, int ND>
 static void launch_walsh_nd(const OpDesc &op, const T *lamu, const T *v, T *q, const Reduce *red, WalshTiles t,
                             hipStream_t s, const DirFuse<T> *fz, const hipEvent_t *ev)
@@ -114,8 +164,9 @@ static void launch_walsh_nd(const OpDesc &op, const T *lamu, const T *v, T *q, c
         const unsigned grid = (unsigned)((op.ny + orows - 1) / orows) * ((op.nx + TCv - 2) / (TCv - 1)) * \
                               ((op.nz + LZ - 1) / LZ);                                                  \
         if (cg1) {                                                                                      \
+            const Reduce fin = cg1_plan(rr, grid);                                                      \
             WALSH_GO(TRv, TCv, H, true, 2)                                                              \
-            launch_reduce_finish(rr, grid, 4, s);                                                       \
+            if (!rr.defer) launch_reduce_finish(fin, grid, 4, s);                                       \
         } else if (fz) {                                                                                \
             WALSH_GO(TRv, TCv, H, true, 1)                                                              \
             launch_reduce_finish(rr, grid, 1, s);                                                       \
@@ -156,8 +207,9 @@ static void launch_walsh_nd(const OpDesc &op, const T *lamu, const T *v, T *q, c
         const unsigned grid = (unsigned)((op.ny + orows - 1) / orows) * ((op.nx + TCv - 2) / (TCv - 1)) * \
                               ((op.nz + LZ - 1) / LZ);                                                  \
         if (cg1) {                                                                                      \
+            const Reduce fin = cg1_plan(rr, grid);                                                      \
             WALSH_GO_SDF(TRv, TCv, H, true, 2)                                                          \
-            launch_reduce_finish(rr, grid, 4, s);                                                       \
+            if (!rr.defer) launch_reduce_finish(fin, grid, 4, s);                                       \
         } else if (red) {                                                                               \
             WALSH_GO_SDF(TRv, TCv, H, true, 0)                                                          \
             launch_reduce_finish(rr, grid, 1, s);                                                       \

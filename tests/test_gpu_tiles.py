@@ -140,3 +140,31 @@ def test_stokes_layer_groups_solve(nz):
         assert rel(m.update_c(2, x), m.update_c(2, xr)) < 1e-6
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("maxit", [1, 2, 16, 17, 37])
+@pytest.mark.parametrize("which", ["elastic", "thermal"])
+@pytest.mark.parametrize("shape", [(4, 5, 3), (24, 24, 24), (33, 64, 50), (48, 90, 61)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_chained_iterations(shape, which, maxit):
+    """On small grids a CG iteration finishes the one before it, in chains that
+    end with the queued batch (16) and with each ring flush.  The iterate after
+    a given number of steps is the oracle's: rounding (1e-16 per step, times a
+    condition below 1e4 and 37 steps) stays below 1e-8; the last shape runs on
+    more blocks than are chained."""
+    rng = np.random.default_rng(sum(shape))
+    img = rng.choice(np.array([0, 255], np.uint8), size=shape)
+    m = H.model(H.ELASTIC, img, [1.0, 0.3, 5.0, 0.2]) if which == "elastic" else H.model(H.THERMAL, img, [1.0, 5.0])
+    if maxit > m.ndof // 2:
+        # 60 unknowns are solved to rounding at step 17 (residual 5e-12); after
+        # that the recurrences divide rounding by rounding, here and in the
+        # oracle, and the iterate drifts along the constants
+        pytest.skip("no more directions left to search")
+    s = H.GpuSolver(m, tol=1e-30, maxit=maxit)
+    try:
+        x, _, st = s.solve(m.rhs(1))
+        xr, _, itr, _ = m.solve(1, tol=1e-30, maxit=maxit)
+        assert int(st.iterations) == itr == maxit
+        assert np.abs(x - xr).max() < 1e-8 * np.abs(xr).max()
+    finally:
+        s.close()

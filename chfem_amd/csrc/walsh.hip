@@ -307,13 +307,14 @@ static double tile_cost(const OpDesc &op, int tr, int tc, int lz)
 }
 
 // The same cost for a batch (FP32), summed over its samples: rounds of blocks
-// become the layer steps of all blocks over the resident slots.  At most 16
-// layers per block: with 32 the last blocks of an uneven batch run alone (8
-// samples of edges 48-80, elastic: 195 ms against 179 with 16).  That batch
-// took 217 ms on 64 x 7 tiles of 32 layers (two row tiles for 65-80 rows);
-// picked: 32 x 8 x 16.  4 samples of edges 20-32: 23.7 -> 10.1 ms (32 x 8 x 4);
-// 3 of 90-130: 515 -> 454 (32 x 8 x 16); 6 of 60-66: 146 -> 135 (64 x 7 x 16);
-// thermal, 8 of 48-80: 28.2 -> 23.8 (64 x 8 x 16; 21.7 with 32 x 8 x 8).
+// become the layer steps of all blocks over the resident slots, and the march
+// of one last block runs alone after them (without that term 32 layers always
+// look best: 8 elastic samples of edges 48-80 take 195 ms with 32 x 8 x 32 and
+// 179 with 16).  Against 64 x 7 x 32 for every batch, device time: that batch
+// 217 -> 179 ms (32 x 8 x 16; 65-80 rows were two row tiles), 4 samples of
+// edges 20-32 23.7 -> 10.1 (32 x 8 x 4), 3 of 90-130 515 -> 454 (32 x 8 x 16),
+// 6 of 60-66 146 -> 135 (64 x 7 x 16), thermal, 8 of 48-80, 28.2 -> 22.4 (64 x
+// 8 x 8); one 256^3 sample keeps 64 x 7 x 32.
 int batch_tile_rule(bool elastic, const batch::Shape *shapes, int nshapes, const std::vector<std::array<int, 3>> &dims,
                     int loads, int &lz_out)
 {
@@ -324,7 +325,7 @@ int batch_tile_rule(bool elastic, const batch::Shape *shapes, int nshapes, const
         const int nt = t.tr == 65 ? 64 * t.tc + 64 : t.tr * t.tc;
         const TileFit f = tile_fit(false, elastic, nt);
         const double vb = sizeof(float) * (elastic ? 3 : 1);
-        for (int lz = 1; lz <= 16; lz *= 2) {
+        for (int lz = 1; lz <= 32; lz *= 2) {
             double nb = 0, steps = 0, longest = 0;
             for (const auto &n : dims) {  // {ny, nx, nz}
                 const double cols = (double)((n[0] + t.rows - 1) / t.rows) * ((n[1] + t.cols - 1) / t.cols) * loads;
@@ -335,8 +336,7 @@ int batch_tile_rule(bool elastic, const batch::Shape *shapes, int nshapes, const
             }
             const double chain = longest * f.step(std::min((double)f.resident, ceil(nb / 256.0)), nt);
             const double all = steps / (256.0 * f.resident) * f.step(f.resident, nt);
-            const double cost = std::max(chain, nb >= 256.0 * f.resident ? all : 0.0) +
-                                f.h * steps * (t.tc + 1) * ((t.rows + 2) + 128.0 / vb) * 1e-6;
+            const double cost = all + chain + f.h * steps * (t.tc + 1) * ((t.rows + 2) + 128.0 / vb) * 1e-6;
             if (cost < least) {
                 least = cost;
                 best = sh;

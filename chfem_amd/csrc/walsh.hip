@@ -127,6 +127,18 @@ static Reduce cg1_plan(Reduce &rr, unsigned grid)
     return fin;
 }
 
+// Layers per block of a launch: those asked for, doubled until the blocks fit
+// the reduction partials.  rows, cols: nodes owned by the tile that is
+// launched.  It can be smaller than the one asked for: 65 x 15 runs as 65 x 7
+// in FP64 and with a density field, other shapes without a kernel as 32 x 8.
+static int layers_per_block(const OpDesc &op, int asked, int rows, int cols)
+{
+    int LZ = asked > 0 ? asked : 16;
+    const long tiles = (long)((op.ny + rows - 1) / rows) * ((op.nx + cols - 1) / cols);
+    while (tiles * ((op.nz + LZ - 1) / LZ) > MAX_PARTIAL_BLOCKS) LZ *= 2;
+    return LZ;
+}
+
 template <typename T, int ND>
 static void launch_walsh_nd(const OpDesc &op, const T *lamu, const T *v, T *q, const Reduce *red, WalshTiles t,
                             hipStream_t s, const DirFuse<T> *fz, const hipEvent_t *ev)
@@ -142,13 +154,6 @@ static void launch_walsh_nd(const OpDesc &op, const T *lamu, const T *v, T *q, c
     // single-kernel CG form: the dinv table given (only launch_apply_cg1
     // sets it; its z output may be absent)
     const bool cg1 = fz && (fz->kinv || (op.sdf.d && fz->dnew));
-    int LZ = t.LZ > 0 ? t.LZ : 16;
-    {
-        // keep the block count within the reduction partials buffer
-        const int tr = t.TR > 0 ? t.TR : 32, tc = t.TC > 0 ? t.TC : 8;
-        const long cols = (long)((op.ny + tr - 2) / (tr - 1)) * ((op.nx + tc - 2) / (tc - 1));
-        while (cols * ((op.nz + LZ - 1) / LZ) > MAX_PARTIAL_BLOCKS) LZ *= 2;
-    }
     // ev: a start and a stop event bound to the k_walsh dispatch itself
     // (hipExtLaunchKernel), so their interval is the kernel's own run time
 #define WALSH_GO(TRv, TCv, H, DOTv, FMv)                                                                \
@@ -161,6 +166,7 @@ static void launch_walsh_nd(const OpDesc &op, const T *lamu, const T *v, T *q, c
 #define WALSH_LAUNCH(TRv, TCv, H)                                                                       \
     {                                                                                                   \
         constexpr int orows = H ? TRv : TRv - 1, nt = TRv * TCv + (H ? 64 : 0);                         \
+        const int LZ = layers_per_block(op, t.LZ, orows, TCv - 1);                                      \
         const unsigned grid = (unsigned)((op.ny + orows - 1) / orows) * ((op.nx + TCv - 2) / (TCv - 1)) * \
                               ((op.nz + LZ - 1) / LZ);                                                  \
         if (cg1) {                                                                                      \
@@ -186,6 +192,7 @@ static void launch_walsh_nd(const OpDesc &op, const T *lamu, const T *v, T *q, c
 #define WALSH_LAUNCH_LEAN(TRv, TCv)                                                                     \
     {                                                                                                   \
         constexpr int nt = TRv * TCv;                                                                   \
+        const int LZ = layers_per_block(op, t.LZ, TRv - 1, TCv - 1);                                    \
         const unsigned grid = (unsigned)((op.ny + TRv - 2) / (TRv - 1)) * ((op.nx + TCv - 2) / (TCv - 1)) * \
                               ((op.nz + LZ - 1) / LZ);                                                  \
         WALSH_GO(TRv, TCv, false, true, 3)                                                              \
@@ -204,6 +211,7 @@ static void launch_walsh_nd(const OpDesc &op, const T *lamu, const T *v, T *q, c
 #define WALSH_LAUNCH_SDF(TRv, TCv, H)                                                                   \
     {                                                                                                   \
         constexpr int orows = H ? TRv : TRv - 1, nt = TRv * TCv + (H ? 64 : 0);                         \
+        const int LZ = layers_per_block(op, t.LZ, orows, TCv - 1);                                      \
         const unsigned grid = (unsigned)((op.ny + orows - 1) / orows) * ((op.nx + TCv - 2) / (TCv - 1)) * \
                               ((op.nz + LZ - 1) / LZ);                                                  \
         if (cg1) {                                                                                      \

@@ -168,3 +168,28 @@ def test_chained_iterations(shape, which, maxit):
         assert np.abs(x - xr).max() < 1e-8 * np.abs(xr).max()
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("solver", [0, 1], ids=["cg", "minres"])
+def test_block_count_of_the_launched_tile(solver, monkeypatch):
+    """A fixed tile that FP64 runs as a smaller one (65x15 as 65x7: 3 tiles of
+    each layer instead of 1): the layers per block keep the launched blocks
+    within the reduction partials.  One layer per block would be 196608 blocks
+    of 4 partials.  The iterate after 20 steps is the default tile's: sums of
+    9e5 terms grouped otherwise differ by less than 1e-12, which 20 steps
+    multiply by less than 1000."""
+    rng = np.random.default_rng(3)
+    m = H.model(H.THERMAL, rng.choice(np.array([0, 255], np.uint8), size=(65536, 1, 14)), [1.0, 5.0])
+    got = []
+    for tile in (None, "65x15x1"):
+        if tile:
+            monkeypatch.setenv("CHFEM_WALSH_TILE", tile)
+        s = H.GpuSolver(m, solver=solver, tol=1e-30, maxit=20)
+        try:
+            x, _, st = s.solve(m.rhs(0))
+            got.append(x)
+            assert int(st.iterations) == 20
+        finally:
+            s.close()
+    assert np.abs(got[0]).max() > 0
+    assert np.abs(got[1] - got[0]).max() < 1e-9 * np.abs(got[0]).max()

@@ -85,8 +85,8 @@ struct Solver {
     float *lamu32 = nullptr;
     bool walsh_ok = false;
     // element-by-element strategy on the Walsh-basis operator: packed node
-    // keys built from the element map (N entries, valid until the map
-    // changes); with a scalar density field the inverse diagonal per node
+    // keys built from the element map (N entries; cudapcgSetImage forms them
+    // again); with a scalar density field the inverse diagonal per node
     uint16_t *ekeys = nullptr;
     size_t ekeys_n = 0;
     bool ekeys_valid = false;
@@ -1984,9 +1984,12 @@ cudapcgFlag_t cudapcgSetX0(cudapcgVar_t *x0, cudapcgFlag_t mustInterpolate)
 cudapcgFlag_t cudapcgSetImage(cudapcgMap_t *img)
 {
     if (!g || !g->model || !img || !g->model->image) return CUDAPCG_FALSE;
-    g->ekeys_valid = false;
-    CHECK_HIP(hipMemcpyAsync(g->model->image, img, g->model->nelem * sizeof(cudapcgMap_t), hipMemcpyHostToDevice,
-                             g->stream));
+    cudapcgModel_t *m = g->model;
+    CHECK_HIP(hipMemcpyAsync(m->image, img, m->nelem * sizeof(cudapcgMap_t), hipMemcpyHostToDevice, g->stream));
+    // node keys formed from the element map: again from this one, here and not
+    // in the next make_ops, which built_model's callers do without
+    if (g->ekeys_valid)
+        launch_keys_from_elements(m->image, g->ekeys, (int)m->nrows, (int)m->ncols, (int)m->nlayers, g->stream);
     CHECK_HIP(hipStreamSynchronize(g->stream));
     g->dinv_valid = false;
     return CUDAPCG_TRUE;

@@ -106,6 +106,36 @@ def test_no_alloc_column_stokes():
     check(na, ref)
 
 
+def test_no_alloc_column_after_another_image():
+    """Element-by-element model: the node keys its kernels read are formed from
+    the element map.  With another map set (cudapcgSetImage) the next column
+    is that of the new material distribution, as hmgUpdateC computes it for a
+    model of the second image."""
+    from chfem_amd.lib import ptr
+    el = {0: (1.0, 0.3), 255: (10.0, 0.2)}
+    first, second = (synthetic.spheres((8, 10, 12), rmin=2, rmax=3, fraction=0.3, seed=s) for s in (31, 32))
+    x = np.random.default_rng(33).standard_normal(3 * first.size)
+    r = H.Resident(first, H.ELASTIC, el, tol=1e-8, strategy=1)
+    try:
+        r.solve(0)
+        elem = synthetic.elem_map(second, [0, 255]).astype(np.uint16)
+        assert r.L.cudapcgSetImage(ptr(elem)) == 1
+        xd, cd = DeviceArray(x), DeviceArray(np.full(r.dim, np.nan))
+        assert r.L.hmgUpdateCNoAlloc(2, xd.ptr, cd.ptr) == 1
+        na = {2: cd.get()}
+        xd.free()
+        cd.free()
+    finally:
+        r.close()
+    r = H.Resident(second, H.ELASTIC, el, tol=1e-8, strategy=1)
+    try:
+        Cf = np.zeros(r.dim * r.dim)
+        assert r.L.hmgUpdateC(2, ptr(x), ptr(Cf)) == 1
+    finally:
+        r.close()
+    check(na, {2: Cf.reshape(r.dim, r.dim)[:, 2].copy()})
+
+
 def test_no_alloc_rejects_without_resident_model():
     from chfem_amd.lib import lib
     L = lib()

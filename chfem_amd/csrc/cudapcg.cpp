@@ -155,12 +155,6 @@ Reduce make_reduce(int fin, int slot)
     r.S = g->S;
     r.fin = fin;
     r.slot = slot;
-    r.guard = 0;
-    r.partials2 = nullptr;
-    r.nb2 = 0;
-    r.chain = r.defer = 0;
-    r.prev = r.Sin = nullptr;
-    r.Sout = nullptr;
     return r;
 }
 

@@ -388,8 +388,7 @@ __global__ void __launch_bounds__(TR *TC) k_ebe_mfma(const T *__restrict__ v, T 
 template <typename T, int TR, int TC>
 static void ebe_mfma_tiles(const OpDesc &op, const T *v, T *q, const Reduce *red, hipStream_t s)
 {
-    Reduce rr = {nullptr, nullptr, 0, 0, 0};
-    if (red) rr = *red;
+    Reduce rr = red ? *red : NO_REDUCE;
     // element layers per block (each block also evaluates the layer below
     // its first one): 32 for FP64 elastic, 16 otherwise (at 256^3: FP64
     // elastic 1.660 -> 1.627 ms with 32; FP32 elastic the same; conduction

@@ -1430,10 +1430,6 @@ logical hmgUpdateCNoAlloc(unsigned int dir, const double *x_dev, double *Ccol_de
     red.partials = sc;
     red.S = sc + NOALLOC_SUMS_OFF;
     red.fin = FIN_STORE;
-    red.slot = 0;
-    red.guard = 0;
-    red.partials2 = nullptr;
-    red.nb2 = 0;
     hipStream_t st = active_stream();
     if (m.analysis == HMG_FLUID) {
         launch_fluid_velocity_sum<double>(dm->op64, x_dev, &red, st);

@@ -54,29 +54,32 @@ enum Finalize {
 };
 
 struct Reduce {
-    double *partials;    // >= (blocks of the launch) * (values reduced) doubles
-    double *S;           // scalar slots
-    int fin;
-    int slot;
+    double *partials = nullptr;  // >= (blocks of the launch) * (values reduced) doubles
+    double *S = nullptr;         // scalar slots
+    int fin = 0;
+    int slot = 0;
     // guarded: the launch and its finishing kernel do nothing once S[S_DONE]
     // is set; a guarded FIN_DELTA finish counts the iteration in S[S_ITER]
     // and sets S[S_DONE] when |r.z| <= S[S_THRESH].  The host can then queue
     // several iterations between synchronisations.
-    int guard;
+    int guard = 0;
     // FIN_STOP_DELTA: the partials an earlier launch left (one value each)
-    const double *partials2;
-    unsigned nb2;
+    const double *partials2 = nullptr;
+    unsigned nb2 = 0;
     // Chained FIN_CG1 (launch_apply_cg1, small grids): the iterations between
     // two points where S has to be current do without the finishing launch;
     // each block of the next iteration adds the partials itself.  chain: the
     // iterations queued since S was current (0: none); defer: the next
     // iteration of this chain finishes this one.
-    int chain, defer;
+    int chain = 0, defer = 0;
     // set by the launcher: the previous iteration's partials (null: S is
     // current) and scalars, and where this launch leaves the scalars it read
-    const double *prev, *Sin;
-    double *Sout;
+    const double *prev = nullptr, *Sin = nullptr;
+    double *Sout = nullptr;
 };
+// a launch without a reduction (a constant expression: it does not compile
+// while a member of Reduce is left without an initial value)
+constexpr Reduce NO_REDUCE;
 // blocks up to which iterations are chained (walsh.hip)
 #define CHAIN_BLOCKS 256
 

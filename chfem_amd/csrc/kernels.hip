@@ -1177,8 +1177,6 @@ static inline int stream_grid(size_t n, size_t elem_bytes)
     return b < 1 ? 1 : (int)b;
 }
 
-static Reduce noreduce() { Reduce r; r.partials = nullptr; r.S = nullptr; r.fin = 0; r.slot = 0; r.guard = 0; r.partials2 = nullptr; r.nb2 = 0; r.chain = r.defer = 0; r.prev = r.Sin = nullptr; r.Sout = nullptr; return r; }
-
 // One block, bound by latency alone: the partials were written by all XCDs,
 // so every read misses this XCD's L2 (about 0.8 us).  The 16 wavefronts share
 // the NV values, each lane issues its 8 reads of a turn before it uses the
@@ -1302,7 +1300,7 @@ void launch_reduce_finish(const Reduce &red, unsigned nb, int nv, hipStream_t s)
 template <typename T>
 void launch_apply(const OpDesc &op, const T *v, T *q, const Reduce *red, hipStream_t s)
 {
-    const Reduce rr = red ? *red : noreduce();
+    const Reduce rr = red ? *red : NO_REDUCE;
     const T *K = (const T *)op.K;
     if (op.physics == PHY_FLUID && op.fkeys) {
         launch_stokes_walsh<T>(op, v, q, red, s);
@@ -1408,7 +1406,7 @@ template <typename T>
 void launch_precond(const T *dinv, const T *v, T *out, size_t n, const Reduce *red, hipStream_t s)
 {
     if (red) LAUNCH_RED(1, (k_precond<T, true>), stream_grid(n, sizeof(T)), s, *red, dinv, v, out, n, *red);
-    else k_precond<T, false><<<stream_grid(n, sizeof(T)), BS, 0, s>>>(dinv, v, out, n, noreduce());
+    else k_precond<T, false><<<stream_grid(n, sizeof(T)), BS, 0, s>>>(dinv, v, out, n, NO_REDUCE);
 }
 
 template <typename T>

@@ -443,8 +443,7 @@ void launch_fluid_node_keys(const OpDesc &op, uint8_t *out, hipStream_t s)
 template <typename T>
 void launch_stokes_walsh(const OpDesc &op, const T *v, T *q, const Reduce *red, hipStream_t s)
 {
-    Reduce rr = {nullptr, nullptr, 0, 0, 0};
-    if (red) rr = *red;
+    Reduce rr = red ? *red : NO_REDUCE;
     constexpr int TR = 32, TC = 8;
     int LZ = op.tile_lz > 0 ? op.tile_lz : STOKES_LZ;
     const long cols = (long)((op.ny + TR - 2) / (TR - 1)) * ((op.nx + TC - 2) / (TC - 1));

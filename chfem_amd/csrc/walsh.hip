@@ -143,8 +143,7 @@ template <typename T, int ND>
 static void launch_walsh_nd(const OpDesc &op, const T *lamu, const T *v, T *q, const Reduce *red, WalshTiles t,
                             hipStream_t s, const DirFuse<T> *fz, const hipEvent_t *ev)
 {
-    Reduce rr = {nullptr, nullptr, 0, 0, 0};
-    if (red) rr = *red;
+    Reduce rr = red ? *red : NO_REDUCE;
     DirFuse<T> f = {nullptr, nullptr, T(0), T(0), 1, 0, nullptr, nullptr, nullptr, 0, T(0), 0, {}, nullptr};
     if (fz) f = *fz;
     f.sdf = op.sdf;

@@ -270,48 +270,72 @@ template void launch_walsh_lean<double>(const OpDesc &, int, const double *, dou
 // 32^3 FP64 conduction iteration took 24.5 us with 16 layers per block, 12
 // blocks on 256 CUs, and takes 13.9 us with 1 or 2), and a grid of many
 // rounds of blocks by what they load, halos included (256^3 FP32 elastic:
-// 332 us with 65x7x32, 382 us with 32x8x16, 369 us with 65x7x8).  The cost of
-// a candidate in us is
-//   rounds of blocks x (LZ + 2) steps x (d + max(L, work-items on a CU x c))
-//   + h x the values its planes load, every column run rounded up by one
-//     128-byte line,
-// with the CU's resident blocks from the kernels' registers and LDS, and d, L,
-// c, h fitted to timed solves (ring, finishing block and launch gaps
-// included) of cubes of 24 to 256 nodes, a 37x41x56 and a 190x251x233 grid,
-// every tile and LZ 1 to 32.  Over those grids the pick is within 3 % of the
-// fastest candidate, 10 % at the worst, where timing every candidate before
-// the first solve cost as much as 30 (256^3) to 150 (32^3) iterations.
+// 347 us with 65x7x32, 394 with 32x8x16).  The cost of a candidate in us is
+//   rounds of blocks x (LZ + 2) steps x (d + work-items on a CU x c)
+//   + h x n / (n + 20) x the million values its planes load, every column run
+//     rounded up by one 128-byte line, n million nodes
+// with the CU's resident blocks from the kernels' registers and LDS, and h, d
+// (by block size) and c (by tile: their halo shares and latencies differ)
+// fitted to which candidate of timed solves was the fastest; halo loads cost
+// little while the vectors stay in the caches, hence n / (n + 20).  Fitted to
+// 65 grids in both precisions and physics, cubes of 16 to 400 nodes and
+// slabs, columns and odd sizes, every tile, LZ 1 to 32: the pick is 0.7 %
+// behind the fastest candidate on average, within 3 % on 94 of 100, at the
+// worst 9 % (50x20x100) and 8 % (400^3), both FP32 elastic.  With one c and d
+// for all tiles, no 65x15 and no 32x16 it was 18 % behind on 192^3 (FP32
+// elastic 166.6 us against 141.0) and 7.5 % on 128^3 (59.8 against 55.7).
+// Timing every candidate before the first solve cost as much as 30 (256^3) to
+// 150 (32^3) iterations.
 struct TileFit {
-    double L, c, d, h;  // see above
-    int resident;       // blocks resident on a CU
-    double step(double on_cu, int nt) const { return d + std::max(L, on_cu * nt * c); }
+    double h, d[3];  // see above; d of blocks of 256, 512 and 1024 work-items
+    double c[7];     // ns per work-item and step, of each tile
 };
+static const int TILES[7][2] = {{32, 8}, {16, 16}, {64, 4}, {64, 8}, {65, 7}, {32, 16}, {65, 15}};
 
-static TileFit tile_fit(bool dbl, bool el, int nt)
+static int size_class(int nt) { return nt <= 256 ? 0 : (nt <= 512 ? 1 : 2); }
+
+// blocks of nt work-items resident on a CU
+static int resident_blocks(bool dbl, bool el, int nt)
 {
-    static const double fit[2][2][4] = {  // [precision][physics] L, c, d, h
-        {{0.400, 0.00059, 0.337, 1.345}, {0.380, 0.00091, 0.699, 4.266}},
-        {{0.839, 0.00134, 0.000, 1.692}, {0.482, 0.00268, 0.920, 4.836}}};
-    // blocks of 256 and of 512 work-items resident on a CU
-    static const int resident[2][2][2] = {{{8, 4}, {5, 2}}, {{6, 3}, {3, 1}}};
-    const double *f = fit[dbl][el];
-    return {f[0], f[1], f[2], f[3], resident[dbl][el][nt > 256]};
+    static const int blocks[2][2][3] = {{{8, 4, 2}, {5, 2, 1}}, {{6, 3, 1}, {3, 1, 1}}};
+    return blocks[dbl][el][size_class(nt)];
+}
+
+// values loaded per step by a tile of rows x cols owned nodes
+static double step_loads(int rows, int cols, double bytes_per_node)
+{
+    return (cols + 2) * ((rows + 2) + 128.0 / bytes_per_node) * 1e-6;
 }
 
 template <typename T>
-static double tile_cost(const OpDesc &op, int tr, int tc, int lz)
+static double tile_cost(const OpDesc &op, int tile, int lz)
 {
-    const bool el = op.physics == PHY_ELASTIC, halo = tr == 65;
-    const int owned = halo ? 64 : tr - 1, nt = halo ? 64 * tc + 64 : tr * tc;
-    const TileFit f = tile_fit(sizeof(T) == 8, el, nt);
-    const double nb = (double)((op.ny + owned - 1) / owned) * ((op.nx + tc - 2) / (tc - 1)) * ((op.nz + lz - 1) / lz);
-    const double slots = 256.0 * f.resident, full = floor(nb / slots), rest = nb - full * slots;
+    static const TileFit fit[2][2] = {  // [precision][physics]
+        {{5.19, {0.503, 0.289, 0.575}, {1.044, 1.268, 0.908, 1.126, 1.180, 1.303, 1.428}},
+         {8.74, {0.772, 0.813, 0.675}, {2.166, 3.064, 2.247, 1.972, 1.890, 2.568, 2.835}}},
+        {{3.87, {0.340, 0.340, 0}, {1.945, 2.040, 1.814, 1.852, 1.838, 2.041, 0}},
+         {17.78, {0.776, 0.776, 0}, {3.967, 4.329, 3.446, 3.957, 3.863, 4.210, 0}}}};
+    const bool dbl = sizeof(T) == 8, el = op.physics == PHY_ELASTIC, halo = TILES[tile][0] == 65;
+    const int rows = halo ? 64 : TILES[tile][0] - 1, tc = TILES[tile][1];
+    const int nt = halo ? 64 * tc + 64 : TILES[tile][0] * tc;
+    const TileFit &f = fit[dbl][el];
+    const double c = f.c[tile] * 1e-3, d = f.d[size_class(nt)];
+    const int resident = resident_blocks(dbl, el, nt);
+    const double tiles = (double)((op.ny + rows - 1) / rows) * ((op.nx + tc - 2) / (tc - 1));
+    if (tiles > MAX_PARTIAL_BLOCKS) return 1e300;
+    const double nb = tiles * ((op.nz + lz - 1) / lz);
+    const double slots = 256.0 * resident, full = floor(nb / slots), rest = nb - full * slots;
     const double steps = std::min(lz, op.nz) + 2;
-    const double chain = full * f.step(f.resident, nt) + (rest > 0 ? f.step(ceil(rest / 256.0), nt) : 0.0);
-    const double vb = sizeof(T) * (el ? 3 : 1);
-    const double loaded = nb * (tc + 1) * ((owned + 2) + 128.0 / vb) * steps * 1e-6;
-    return chain * steps + f.h * loaded;
+    const double chain = full * (d + resident * nt * c) + (rest > 0 ? d + ceil(rest / 256.0) * nt * c : 0.0);
+    const double n = (double)op.ny * op.nx * op.nz * 1e-6;
+    return steps * (chain + f.h * n / (n + 20.0) * nb * step_loads(rows, tc - 1, sizeof(T) * (el ? 3 : 1)));
 }
+
+struct BatchFit {
+    double L, c, d, h;
+    int resident;
+    double step(double on_cu, int nt) const { return d + std::max(L, on_cu * nt * c); }
+};
 
 // The same cost for a batch (FP32), summed over its samples: rounds of blocks
 // become the layer steps of all blocks over the resident slots, and the march
@@ -330,7 +354,8 @@ int batch_tile_rule(bool elastic, const batch::Shape *shapes, int nshapes, const
     for (int sh = 0; sh < nshapes; sh++) {
         const batch::Shape &t = shapes[sh];
         const int nt = t.tr == 65 ? 64 * t.tc + 64 : t.tr * t.tc;
-        const TileFit f = tile_fit(false, elastic, nt);
+        const BatchFit f = elastic ? BatchFit{0.380, 0.00091, 0.699, 4.266, resident_blocks(false, true, nt)}
+                                   : BatchFit{0.400, 0.00059, 0.337, 1.345, resident_blocks(false, false, nt)};
         const double vb = sizeof(float) * (elastic ? 3 : 1);
         for (int lz = 1; lz <= 32; lz *= 2) {
             double nb = 0, steps = 0, longest = 0;
@@ -357,20 +382,18 @@ int batch_tile_rule(bool elastic, const batch::Shape *shapes, int nshapes, const
 template <typename T>
 WalshTiles walsh_tile_rule(const OpDesc &op, int lean)
 {
-    static const int shapes[][2] = {{32, 8}, {16, 16}, {64, 4}, {64, 8}, {65, 7}};
     WalshTiles best = {32, 8, 16};
     double least = 1e300;
-    for (const auto &sh : shapes) {
-        if (lean && sh[0] != 32) continue;
-        if (op.sdf.d && sh[0] != 32 && sh[0] != 65) continue;
-        // (16-row FP32 columns are 204-byte runs: the fit prefers them at
-        // 160^3, where they measured 11 % slower than 64x8)
-        if (sh[0] == 16 && sizeof(T) == 4) continue;
+    for (int tile = 0; tile < 7; tile++) {
+        const int tr = TILES[tile][0], tc = TILES[tile][1];
+        if (lean && tile != 0) continue;
+        if (op.sdf.d && tile != 0 && tile != 4) continue;
+        if (sizeof(T) == 8 && tc == 15) continue;  // does not fit in LDS
         for (int lz = 1; lz <= 32; lz *= 2) {
-            const double c = tile_cost<T>(op, sh[0], sh[1], lz);
+            const double c = tile_cost<T>(op, tile, lz);
             if (c < least) {
                 least = c;
-                best = {sh[0], sh[1], lz};
+                best = {tr, tc, lz};
             }
         }
     }

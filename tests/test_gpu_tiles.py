@@ -44,6 +44,41 @@ def test_rule_tile_solves(shape, which, precision):
         s.close()
 
 
+@pytest.mark.parametrize("which,precision,shape,tile", [
+    ("elastic", 1, (71, 64, 85), (65, 15, 2)),
+    ("elastic", 1, (113, 32, 29), (32, 16, 2)),
+    ("thermal", 1, (67, 31, 50), (32, 16, 2)),
+    ("thermal", 0, (41, 49, 89), (32, 16, 2)),
+    ("elastic", 0, (41, 49, 89), (32, 16, 2)),
+    ("thermal", 1, (38, 33, 48), (16, 16, 2)),
+], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_rule_picks(which, precision, shape, tile, monkeypatch):
+    """Grids on which the rule takes 65x15, 32x16 and, in FP32, 16x16 tiles: the
+    pick, and the iterate after 20 steps against a 32x8x16 tile's.  Sums grouped otherwise and the
+    layers of a block begun elsewhere change single roundings (6e-8 in FP32,
+    1e-16 in FP64), which 20 steps multiply by less than 1000."""
+    rng = np.random.default_rng(sum(shape))
+    img = rng.choice(np.array([0, 255], np.uint8), size=shape)
+    m = H.model(H.ELASTIC, img, [1.0, 0.3, 5.0, 0.2]) if which == "elastic" else H.model(H.THERMAL, img, [1.0, 5.0])
+    monkeypatch.setenv("CHFEM_RELIABLE_DROP", "1e-30")
+    got = []
+    for env in (None, "32x8x16"):
+        if env:
+            monkeypatch.setenv("CHFEM_WALSH_TILE", env)
+        s = H.GpuSolver(m, precision=precision, tol=1e-30, maxit=20)
+        try:
+            x, _, st = s.solve(m.rhs(1))
+            t = np.zeros(3, dtype=np.int32)
+            assert s.L.cudapcgGetOperatorTile(precision, s.ptr(t)) == 1
+            assert tuple(t) == (tile if env is None else (32, 8, 16))
+            assert int(st.iterations) == 20
+            got.append(x)
+        finally:
+            s.close()
+    scale = np.abs(got[1]).max()
+    assert scale > 0 and np.abs(got[0] - got[1]).max() < (6e-5 if precision else 1e-10) * scale
+
+
 @pytest.mark.parametrize("env", [None, "mfma"], ids=["default", "matrix-cores"])
 @pytest.mark.parametrize("which", ["elastic", "thermal"])
 @pytest.mark.parametrize("shape", [(3, 2, 4), (9, 70, 40), (17, 33, 65)], ids=lambda s: "x".join(map(str, s)))

@@ -331,46 +331,44 @@ static double tile_cost(const OpDesc &op, int tile, int lz)
     return steps * (chain + f.h * n / (n + 20.0) * nb * step_loads(rows, tc - 1, sizeof(T) * (el ? 3 : 1)));
 }
 
-struct BatchFit {
-    double L, c, d, h;
-    int resident;
-    double step(double on_cu, int nt) const { return d + std::max(L, on_cu * nt * c); }
-};
-
-// The same cost for a batch (FP32), summed over its samples: rounds of blocks
-// become the layer steps of all blocks over the resident slots, and the march
-// of one last block runs alone after them (without that term 32 layers always
-// look best: 8 elastic samples of edges 48-80 take 195 ms with 32 x 8 x 32 and
-// 179 with 16).  Against 64 x 7 x 32 for every batch, device time: that batch
-// 217 -> 179 ms (32 x 8 x 16; 65-80 rows were two row tiles), 4 samples of
-// edges 20-32 23.7 -> 10.1 (32 x 8 x 4), 3 of 90-130 515 -> 454 (32 x 8 x 16),
-// 6 of 60-66 146 -> 135 (64 x 7 x 16), thermal, 8 of 48-80, 28.2 -> 22.4 (64 x
-// 8 x 8); one 256^3 sample keeps 64 x 7 x 32.
+// The same for a batch (FP32), summed over its samples: rounds of blocks
+// become the layer steps of all blocks over the resident slots, and w marches
+// of one last block run alone after them.  Fitted to 36 batches of 1 to 32
+// samples of 24 to 288 nodes: the pick is 0.8 % behind the fastest of the 18
+// candidates on average and 8 % at the worst (one 96^3 elastic sample), and
+// on none slower than 64 x 7 x 32 for every batch (8 elastic samples of edges
+// 48-80 217 -> 179 ms, 4 of 20-32 23.7 -> 10.1, 3 of 90-130 515 -> 454).  The
+// coefficients of the rule before made conduction of one 256^3 sample 5 %
+// slower than that, one of 233x190x251 6 % (64 x 7 x 16).
 int batch_tile_rule(bool elastic, const batch::Shape *shapes, int nshapes, const std::vector<std::array<int, 3>> &dims,
                     int loads, int &lz_out)
 {
+    struct BatchFit { double d, h, w, c[3]; };
+    static const BatchFit fit[2] = {{2.72, 8.06, 0.216, {0.234, 0.289, 0.223}},
+                                    {1.53, 12.6, 0.518, {0.246, 0.501, 0.286}}};
+    const BatchFit &f = fit[elastic];
     int best = 0;
-    double least = 1e300;
-    for (int sh = 0; sh < nshapes; sh++) {
+    double least = 1e300, n = 0;
+    for (const auto &g : dims) n += (double)g[0] * g[1] * g[2] * loads * 1e-6;
+    for (int sh = 0; sh < nshapes && sh < 3; sh++) {
         const batch::Shape &t = shapes[sh];
         const int nt = t.tr == 65 ? 64 * t.tc + 64 : t.tr * t.tc;
-        const BatchFit f = elastic ? BatchFit{0.380, 0.00091, 0.699, 4.266, resident_blocks(false, true, nt)}
-                                   : BatchFit{0.400, 0.00059, 0.337, 1.345, resident_blocks(false, false, nt)};
-        const double vb = sizeof(float) * (elastic ? 3 : 1);
+        const int resident = resident_blocks(false, elastic, nt);
+        auto step = [&](double on_cu) { return f.d + on_cu * nt * f.c[sh] * 1e-3; };
         for (int lz = 1; lz <= 32; lz *= 2) {
             double nb = 0, steps = 0, longest = 0;
-            for (const auto &n : dims) {  // {ny, nx, nz}
-                const double cols = (double)((n[0] + t.rows - 1) / t.rows) * ((n[1] + t.cols - 1) / t.cols) * loads;
-                const int chunks = (n[2] + lz - 1) / lz;
+            for (const auto &g : dims) {  // {ny, nx, nz}
+                const double cols = (double)((g[0] + t.rows - 1) / t.rows) * ((g[1] + t.cols - 1) / t.cols) * loads;
+                const int chunks = (g[2] + lz - 1) / lz;
                 nb += cols * chunks;
-                steps += cols * (n[2] + 2 * chunks);
-                longest = std::max(longest, std::min(lz, n[2]) + 2.0);
+                steps += cols * (g[2] + 2 * chunks);
+                longest = std::max(longest, std::min(lz, g[2]) + 2.0);
             }
-            const double chain = longest * f.step(std::min((double)f.resident, ceil(nb / 256.0)), nt);
-            const double all = steps / (256.0 * f.resident) * f.step(f.resident, nt);
-            const double cost = all + chain + f.h * steps * (t.tc + 1) * ((t.rows + 2) + 128.0 / vb) * 1e-6;
-            if (cost < least) {
-                least = cost;
+            const double all = steps / (256.0 * resident) * step(resident);
+            const double last = f.w * longest * step(std::min((double)resident, ceil(nb / 256.0)));
+            const double loads_cost = f.h * n / (n + 400.0) * steps * step_loads(t.rows, t.cols, elastic ? 12 : 4);
+            if (all + last + loads_cost < least) {
+                least = all + last + loads_cost;
                 best = sh;
                 lz_out = lz;
             }

@@ -228,3 +228,29 @@ def test_block_count_of_the_launched_tile(solver, monkeypatch):
             s.close()
     assert np.abs(got[0]).max() > 0
     assert np.abs(got[1] - got[0]).max() < 1e-9 * np.abs(got[0]).max()
+
+
+@pytest.mark.parametrize("solver", [0, 1], ids=["cg", "minres"])
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("which", ["elastic", "thermal"])
+def test_timed_tiles(which, precision, solver, monkeypatch):
+    """CHFEM_WALSH_TILE=auto: the timed choice of tile and loop form, and the
+    solve that follows (residual 1e-9, condition below 100: 1e-7 in C).  The
+    rule's tile is a candidate: on this grid tiles of 16 layers take over
+    twice as long per FP64 elastic iteration."""
+    monkeypatch.setenv("CHFEM_WALSH_TILE", "auto")
+    rng = np.random.default_rng(24)
+    img = rng.choice(np.array([0, 255], np.uint8), size=(24, 24, 24))
+    m = H.model(H.ELASTIC, img, [1.0, 0.3, 5.0, 0.2]) if which == "elastic" else H.model(H.THERMAL, img, [1.0, 5.0])
+    s = H.GpuSolver(m, solver=solver, precision=precision, tol=1e-9)
+    try:
+        x, ok, _ = s.solve(m.rhs(0))
+        xr, okr, _, _ = m.solve(0, tol=1e-9)
+        t = np.zeros(3, dtype=np.int32)
+        assert s.L.cudapcgGetOperatorTile(precision, s.ptr(t)) == 1
+        assert ok and okr and rel(m.update_c(0, x), m.update_c(0, xr)) < 1e-7
+        assert s.L.cudapcgGetLoopForm(precision) in (1, 2)
+        if which == "elastic" and precision == 0 and solver == 0:
+            assert t[2] <= 4, t
+    finally:
+        s.close()

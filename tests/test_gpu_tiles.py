@@ -137,6 +137,39 @@ def test_density_solves(shape, which, solver, precision):
 
 
 @pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("tile", ["32x8x5", "65x7x5"])
+@pytest.mark.parametrize("which", ["elastic", "thermal"])
+def test_density_tiles(which, tile, precision, monkeypatch):
+    """Both tile shapes of the density kernels with several layers per block,
+    on a grid ragged in every direction (two tiles along the rows, a last
+    chunk of one layer), densities independent from element to element: the
+    operator in the precision of the loop, and a solve (tolerances as in
+    test_density_solves; FP32 rounds sums over 8 elements)."""
+    monkeypatch.setenv("CHFEM_WALSH_TILE", tile)
+    rng = np.random.default_rng(70)
+    img = rng.choice(np.array([0, 255], np.uint8), size=(11, 70, 23))
+    m = H.model(H.ELASTIC, img, [1.0, 0.3, 1.0, 0.2]) if which == "elastic" else H.model(H.THERMAL, img, [1.0, 2.0])
+    d = rng.integers(0, 65536, size=m.N).astype(np.uint16)
+    lo, hi = 0.01, 1.0
+    m.set_element_scale(d.astype(np.float64) * (1.0 / 65535.0) * (hi - lo) + lo)
+    s = H.GpuSolver(m, strategy=1, precision=precision, tol=1e-9)
+    try:
+        assert s.L.cudapcgSetParametricDensityField(s.ptr(d), lo, hi) == 1
+        v = rng.standard_normal(m.ndof).astype(np.float32)
+        q = m.apply(v.astype(np.float64), strategy=1)
+        if precision:
+            assert np.abs(s.apply32(v) - q).max() < 1e-5 * np.abs(q).max()
+        else:
+            assert rel(s.apply(v.astype(np.float64)), q) < 1e-12
+        x, ok, _ = s.solve(m.rhs(0))
+        xr, okr, _, _ = m.solve(0, tol=1e-9, strategy=1)
+        assert ok and okr
+        assert rel(m.update_c(0, x), m.update_c(0, xr)) < 1e-6
+    finally:
+        s.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
 @pytest.mark.parametrize("shape", [(2, 5, 9), (3, 33, 16), (7, 62, 30), (10, 100, 63), (16, 14, 31)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_stokes_layer_groups(shape, precision, monkeypatch):

@@ -112,7 +112,7 @@ def test_cli_reference_harness_recursive_guess(tmp_path, case):
 
 
 def test_cli_elastic_ebe_golden(tmp_path):
-    """Elastic Y on the element-by-element operator (matrix cores), without
+    """Elastic Y on the element-by-element strategy, without
     the recursive guess, against the golden column."""
     nf, raw = copy_inputs(tmp_path, "elastic_ggg40_100.nf", "ggg40_100.raw")
     out = str(tmp_path / "C.bin")

@@ -3,12 +3,13 @@ fixtures tests/golden/make_configs.py wrote from the CPU FP64 oracle:
 
 * C1  32^3 Gaussian-random-field conductivity: FP64 and mixed precision,
       NBN and EBE, against the oracle's 3x3 tensor (tol 1e-10);
-* C2  128^3 sphere elasticity: FP64 and mixed, NBN and EBE (matrix cores),
-      against the oracle's 6x6 tensor (tol 1e-9);
+* C2  128^3 sphere elasticity: FP64 and mixed, NBN and EBE (the Walsh-basis
+      operator on node keys formed from the element map), against the
+      oracle's 6x6 tensor (tol 1e-9);
 * headline 256^3 sphere elasticity: FP64 against the oracle's X and YZ
       columns (tol 1e-8), and the benchmark's own method (mixed precision at
-      tol 1e-5 from the zero guess and from a learned guess, autotuned tiles)
-      against them within the metric's 1e-4;
+      tol 1e-5 from the zero guess and from a learned guess) against them
+      within the metric's 1e-4;
 * C3  256^3 Stokes permeability: the library's fluid keys, DOF numbering,
       DOF->node map and border keys hash to the oracle's; MINRES in FP64 and
       mixed precision give a symmetric tensor with a positive diagonal, the
@@ -145,9 +146,9 @@ def test_headline_fp64_vs_oracle(headline):
 @pytest.mark.timeout(900)
 def test_headline_benchmark_method_vs_oracle(headline):
     """The benchmark's method: all 6 load cases resident, mixed precision at
-    tolerance 1e-5 with the autotuned tiles, from the zero guess and from a
-    learned initial guess trained on a reduced set of 64^3 images of the same
-    recipe; the columns the oracle solved within the metric's 1e-4."""
+    tolerance 1e-5, from the zero guess and from a learned initial guess
+    trained on a reduced set of 64^3 images of the same recipe; the columns
+    the oracle solved within the metric's 1e-4."""
     from chfem_amd import guess
     from chfem_amd.guessbench import solve_resident
     img, fx = headline

@@ -134,14 +134,16 @@ def test_golden_sdf(case, tmp_path):
     assert np.abs(C[:, d] - ref[:, d]).max() / np.abs(ref).max() < 1e-4
 
 
-@pytest.mark.parametrize("kernel", ["mfma", "atomic"])
+@pytest.mark.parametrize("kernel", ["mfma", "atomic", "default"])
 @pytest.mark.parametrize("which", ["thermal", "elastic"])
 def test_sdf_vs_oracle(which, kernel, monkeypatch):
     """Element-by-element operator, Jacobi, RHS and solve with a random 16-bit
-    density field against the oracle with the same element scales."""
+    density field against the oracle with the same element scales: on the
+    matrix cores, with the atomic element kernel, and on the Walsh-basis
+    operator (default)."""
     from chfem_amd.lib import lib, ptr
-    if kernel == "atomic":
-        monkeypatch.setenv("CHFEM_EBE", "atomic")
+    if kernel != "default":
+        monkeypatch.setenv("CHFEM_EBE", kernel)
     rng = np.random.default_rng(61)
     img = rng.choice(np.array([0, 255], dtype=np.uint8), size=(9, 17, 12))
     if which == "thermal":
@@ -164,8 +166,8 @@ def test_sdf_vs_oracle(which, kernel, monkeypatch):
         assert relmax(m.update_c(m.cdim - 1, x), m.update_c(m.cdim - 1, xr)) < 1e-7
     finally:
         s.close()
-    # the FP32 operator of mixed precision (the matrix-core kernel's 4x4
-    # block form scales each element's gathered values) on an
+    # the FP32 operator of mixed precision (on the matrix cores the 4x4x1
+    # block form, which scales each element's gathered values) on an
     # FP32-representable input
     s = H.GpuSolver(m, strategy=1, precision=1, tol=1e-9)
     try:

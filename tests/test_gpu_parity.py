@@ -218,9 +218,9 @@ def test_mixed_precision_elastic(ragged_elastic):
 @pytest.mark.parametrize("which", ["elastic", "thermal"])
 def test_walsh_operator_tiles(which, tile, shape, monkeypatch):
     """Walsh-basis operators (isotropic elastic, conduction) on ragged, tiny
-    and multi-chunk grids for every tile shape, NBN and EBE (atomic-form
-    strategy, which also routes to the Walsh kernel), against the oracle's
-    dense local matrices."""
+    and multi-chunk grids for every tile shape, NBN and EBE (CHFEM_EBE=atomic:
+    on the element map, not on node keys formed from it), against the
+    oracle's dense local matrices."""
     monkeypatch.setenv("CHFEM_WALSH_TILE", tile)
     monkeypatch.setenv("CHFEM_EBE", "atomic")
     img = three_phase(shape, 21)
@@ -331,16 +331,22 @@ def test_mfma_4x4_layout():
     np.testing.assert_allclose(got.transpose(0, 2, 1), Db, rtol=1e-6, atol=1e-6)
 
 
-@pytest.mark.parametrize("kernel", ["mfma", "mfma-32x8", "atomic"])
+@pytest.mark.parametrize("kernel", ["mfma", "mfma-32x8", "atomic", "atomic-elements", "default"])
 @pytest.mark.parametrize("which", ["thermal", "elastic"])
 @pytest.mark.parametrize("nphase", [1, 4])
 def test_ebe_kernels(kernel, which, nphase, monkeypatch):
-    """EBE operator on the matrix cores (16x16 element tiles by default, and
-    32x8) and the reference-style element kernel with atomics, with 1 and 4
-    materials on a grid of several blocks in every direction, FP64 and FP32
-    against the oracle."""
-    if kernel == "atomic":
+    """EBE operators with 1 and 4 materials on a grid of several blocks in every
+    direction, FP64 and FP32 against the oracle: on the matrix cores (16x16
+    element tiles, FP32 in 4x4x1 blocks, and 32x8 tiles), the Walsh-basis
+    operator on the element map (CHFEM_EBE=atomic), the reference-style element
+    kernel with atomics (the same with the generic operators), and the default,
+    the Walsh-basis operator on node keys formed from the element map."""
+    if kernel == "mfma":
+        monkeypatch.setenv("CHFEM_EBE", "mfma")
+    if kernel.startswith("atomic"):
         monkeypatch.setenv("CHFEM_EBE", "atomic")
+    if kernel == "atomic-elements":
+        monkeypatch.setenv("CHFEM_OPERATOR", "generic")
     if kernel == "mfma-32x8":
         monkeypatch.setenv("CHFEM_EBE_TILE", "32x8")
     rng = np.random.default_rng(51 + nphase)

@@ -75,7 +75,7 @@ struct Solver {
     // vector kernels, FP64 and FP32
     double *kinv64 = nullptr;
     float *kinv32 = nullptr;
-    // operator tiles chosen by the autotuner (rows, columns, layers per block)
+    // operator tiles chosen by the timed sweep (rows, columns, layers per block)
     bool autotune = false, tuned = false;
     int tile64[3] = {32, 8, 16}, tile32[3] = {32, 8, 16};
     // CG loop form per precision (see fuse_mode_env)
@@ -429,9 +429,11 @@ static int make_ops()
     // Element-by-element strategy: where the Walsh-basis operator takes the
     // local matrices it computes the same product with a sixth of the
     // matrix-core kernel's operations and the single-kernel iterations come
-    // with it (CHFEM_EBE or CHFEM_EBE_TILE set: the element kernels).
-    // Without a density field the element map is packed into node keys and
-    // the model runs as a node-by-node one.
+    // with it.  CHFEM_EBE or CHFEM_EBE_TILE set: the matrix-core kernel;
+    // CHFEM_EBE=atomic: the Walsh-basis operator on the element map, with a
+    // density field the atomic element kernel.  By default, without a density
+    // field, the element map is packed into node keys and the model runs as a
+    // node-by-node one.
     const char *esel = getenv("CHFEM_EBE");
     const bool ebe_kernels = esel || getenv("CHFEM_EBE_TILE");
     o.ebe_matrix = o.ebe && ebe_kernels;

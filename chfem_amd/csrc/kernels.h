@@ -123,10 +123,10 @@ struct OpDesc {
     // with a scalar density field on the Walsh-basis operator: selects its
     // single-kernel CG form
     const void *dnode;
-    // EBE with local matrices that the Walsh-basis operator does not take (or
-    // CHFEM_EBE / CHFEM_EBE_TILE set): 1 selects the reference-style element
-    // kernel with atomics instead of the matrix-core kernel (ebe_mfma.hip; up
-    // to 4 materials)
+    // EBE: 1 (CHFEM_EBE=atomic) keeps the model off the matrix-core kernel
+    // (ebe_mfma.hip; up to 4 materials).  It then runs the Walsh-basis operator
+    // on the element map where lamu is set, and the reference-style element
+    // kernel with atomics otherwise (other matrices, a density field).
     int ebe_atomic;
     // EBE: 1 keeps the matrix-core kernel where lamu would allow the
     // Walsh-basis operator

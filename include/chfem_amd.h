@@ -195,13 +195,15 @@ int chfemMfmaCheck4(const float *A, const float *B, float *D);
 cudapcgFlag_t cudapcgSetKernelTiming(cudapcgFlag_t on);
 cudapcgFlag_t cudapcgGetKernelTiming(double *op_ms_total, unsigned int *op_launches);
 /* Walsh-basis operator tile in use for a precision (rows, columns and node
- * layers per block), as fixed by CHFEM_WALSH_TILE or chosen by the
- * autotuner before the first solve. */
+ * layers per block): picked from the grid by a fitted cost, fixed by
+ * CHFEM_WALSH_TILE=TRxTCxLZ, or with CHFEM_WALSH_TILE=auto the fastest of a
+ * timed sweep before the first solve. */
 cudapcgFlag_t cudapcgGetOperatorTile(cudapcgFlag_t precision, int *tile);
 /* Form of the Jacobi-PCG loop on the Walsh-basis operators for a precision:
  * 0 separate kernels, 1 direction and iterate updates inside the operator
- * plus a z update kernel, 2 single-kernel iterations; fixed by
- * CHFEM_FUSE_DIR or chosen by the autotuner (-1 without a solver). */
+ * plus a z update kernel, 2 single-kernel iterations (the default); fixed
+ * by CHFEM_FUSE_DIR, or chosen by the sweep of CHFEM_WALSH_TILE=auto (-1
+ * without a solver). */
 int cudapcgGetLoopForm(cudapcgFlag_t precision);
 /* Same counters for the last hmgSolveResident / hmgSolveHomogenization. */
 cudapcgFlag_t hmgGetKernelTiming(double *op_ms_total, unsigned int *op_launches);

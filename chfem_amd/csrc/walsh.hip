@@ -307,8 +307,9 @@ static double step_loads(int rows, int cols, double bytes_per_node)
     return (cols + 2) * ((rows + 2) + 128.0 / bytes_per_node) * 1e-6;
 }
 
+// (lean: the memory-lean forms, whose steps have twice the latency d)
 template <typename T>
-static double tile_cost(const OpDesc &op, int tile, int lz)
+static double tile_cost(const OpDesc &op, int tile, int lz, int lean)
 {
     static const TileFit fit[2][2] = {  // [precision][physics]
         {{5.19, {0.503, 0.289, 0.575}, {1.044, 1.268, 0.908, 1.126, 1.180, 1.303, 1.428}},
@@ -319,7 +320,7 @@ static double tile_cost(const OpDesc &op, int tile, int lz)
     const int rows = halo ? 64 : TILES[tile][0] - 1, tc = TILES[tile][1];
     const int nt = halo ? 64 * tc + 64 : TILES[tile][0] * tc;
     const TileFit &f = fit[dbl][el];
-    const double c = f.c[tile] * 1e-3, d = f.d[size_class(nt)];
+    const double c = f.c[tile] * 1e-3, d = (lean ? 2 : 1) * f.d[size_class(nt)];
     const int resident = resident_blocks(dbl, el, nt);
     const double tiles = (double)((op.ny + rows - 1) / rows) * ((op.nx + tc - 2) / (tc - 1));
     if (tiles > MAX_PARTIAL_BLOCKS) return 1e300;
@@ -387,8 +388,10 @@ WalshTiles walsh_tile_rule(const OpDesc &op, int lean)
         if (lean && tile != 0) continue;
         if (op.sdf.d && tile != 0 && tile != 4) continue;
         if (sizeof(T) == 8 && tc == 15) continue;  // does not fit in LDS
-        for (int lz = 1; lz <= 32; lz *= 2) {
-            const double c = tile_cost<T>(op, tile, lz);
+        // (memory-lean forms: 32 layers were slower than 16 on every grid, up
+        // to 6 % at 192^3 FP64 elastic, 447 us per CG3 iteration against 421)
+        for (int lz = 1; lz <= (lean ? 16 : 32); lz *= 2) {
+            const double c = tile_cost<T>(op, tile, lz, lean);
             if (c < least) {
                 least = c;
                 best = {tr, tc, lz};

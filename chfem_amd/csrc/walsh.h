@@ -545,7 +545,7 @@ __device__ __forceinline__ TileSums walsh_tile(const T *__restrict__ v, T *__res
         // them too (in bounds, unused): every step then has the same loads
         // and none is pending across the loop's back edge.
         const uint32_t kcur = kraw;
-        if constexpr (!LEAN) mk = mat_key(lw1);
+        if constexpr (!(LEAN && ND == 1)) mk = mat_key(lw1);
         dk = dens_key(lw1);
         // CG1: dinv and diag of the owned node (its key is the element's,
         // loaded a step ahead), read after this layer's elements
@@ -559,11 +559,12 @@ __device__ __forceinline__ TileSums walsh_tile(const T *__restrict__ v, T *__res
                 dgo[a] = fz.kinv ? fz.kinv[(size_t)65536 * ND + ND * kcur + a] : T(1);
                 zo[a] = fz.lean == 3 ? q[on + a] : T(0);
             }
-            // (after the branches above: loaded before them, the key's zero
-            // extension is an instruction of its own among the elements and
-            // waits for the load there; CG3 conduction at 128^3 64.0 us per
-            // iteration, 59.5 here)
-            mk = mat_key(lw1);
+            // (conduction, after the branches above: loaded before them, the
+            // key's zero extension is an instruction of its own among the
+            // elements and waits for the load there; CG3 at 128^3 64.0 us per
+            // iteration, 59.5 here.  The elastic forms are 1 % faster with
+            // the early load.)
+            if constexpr (ND == 1) mk = mat_key(lw1);
         }
         // owned node's d (and, CG1, its updated z), read from the planes of
         // layer l here, before any work-item replaces them (after the
